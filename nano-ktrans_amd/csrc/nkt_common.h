@@ -285,6 +285,16 @@ __device__ __forceinline__ void wait_vmem() {
   __asm__ volatile("" ::: "memory");
 }
 
+// Waits until at most N of this wave's vector-memory loads are outstanding
+// (they return in order: all but the newest N have landed).
+template <int N>
+__device__ __forceinline__ void wait_vmem_but() {
+  static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit count");
+  __asm__ volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | (N >> 4) << 14);
+  __asm__ volatile("" ::: "memory");
+}
+
 // ---------------------------------------------------------------------------
 // MFMA wrappers (gfx950)
 //   16x16x32 bf16: lane l supplies A[l%16][8*(l/16) .. +7] and

@@ -10,9 +10,9 @@
 //   * gemm2_i8_kernel (int8): 4 waves, three-stage pipeline of 64-wide K
 //     stages (tokens direct-to-LDS, weights in a register ring), gate_up on
 //     the fp16 matrix cores;
-//   * gemm2_i4_kernel (int4 g128): 8 waves, three-stage pipeline of 128-wide
+//   * gemm2_i4_kernel (int4 g128): 4 waves, three-stage pipeline of 128-wide
 //     K stages (tokens, scales and group sums direct-to-LDS, weights in a
-//     register ring);
+//     ring of two register stages);
 //   * gemm2_kernel (bf16 weights, and int8 / int4 operands past the
 //     pipelines' 32-bit buffer offsets): the register-staged form below.
 // The two pipelines also hold copies that compute only the first 16 / 32
@@ -823,38 +823,47 @@ bool gemm2_supported(int wf, int phase, int N, int K, int I) {
 }
 
 // ---------------------------------------------------------------------------
-// int4 g128 weights, three-stage pipeline.  Same tile, waves (8, two 16-row
-// tiles each), work order, MFMA and scaling sequence and epilogue as
-// gemm2_kernel<WF_I4, ...> (so the results are the same bit for bit); K
-// advances one 128-wide scale group per stage:
+// int4 g128 weights, three-stage pipeline.  Same tile, work order and scaling
+// sequence as gemm2_kernel<WF_I4, ...>; 4 waves of four 16-row tiles each,
+// two workgroups per CU; K advances one 128-wide scale group per stage:
 //   * tokens: 64 positions x 256 B per stage reach one of three LDS buffers
-//     by direct-to-LDS buffer loads (16 loads of 4 positions, 2 per wave);
+//     by direct-to-LDS buffer loads (16 loads of 4 positions, 4 per wave);
 //     lane l carries position 4 i + l / 16 into slot l % 16 of that
 //     position's row, fetched from chunk (l % 16) ^ (position % 16), so the
 //     MFMA operand reads of 16 consecutive positions cover all 64 banks;
-//   * each wave's two 1 KiB weight blocks go by buffer loads straight into a
-//     three-deep register ring; their bf16 scales (lanes 0-15, 4 bytes
+//   * each wave's four 1 KiB weight blocks go by buffer loads straight into
+//     one of two register stages; their bf16 scales (lanes 0-31, 4 bytes
 //     each) and the 64 positions' activation group sums (4 bytes per lane)
 //     reach the wave's own slice of a small LDS buffer by direct-to-LDS
 //     loads;
-//   * step x: wait for this wave's loads of stage x (all but the newest 6,
+//   * step x: wait for this wave's loads of stage x (all but the newest 10,
 //     the loads of stage x + 1), one LDS-only barrier (every wave is also
-//     done reading stage x - 1's buffers), start stage x + 2's loads into
-//     those buffers and that ring slot, then stage x: four MFMAs per (row
-//     tile, column tile) into a temporary that starts at the code offset,
-//     the 8 temporaries advancing together, then scaled into the
+//     done reading stage x - 1's buffers), start stage x + 2's token loads
+//     into those buffers, dequantise stage x's weights, start stage x + 2's
+//     weight loads into the registers that frees, then column tile by column
+//     tile: four MFMAs per row tile into a temporary that starts at the code
+//     offset, the 4 temporaries advancing together, then scaled into the
 //     accumulators.
+// What bounds it: neither HBM nor one unit, but the waits a stage's barrier
+// and an item's start and end leave.  Four waves of 64 rows read each token
+// fragment from LDS half as often as eight waves of 32, and fit two
+// workgroups per CU (251 VGPRs at 2 waves per SIMD; eight waves of 210
+// allowed one), so one computes while the other waits.  Measured, eight
+// waves -> this: Mixtral T = 2048 gate_up 1081 -> 933 us (890 -> 1031
+// TFLOP/s), down 588 -> 536; Qwen3 T = 2048 gate_up 185 -> 164, down 124 ->
+// 96; Qwen3 T = 203 (narrow copies) gate_up 47.7 -> 44.4, down 33.4 -> 27.1.
 // Loads past the last stage take an out-of-range buffer offset (no
-// traffic), so every step issues the same 6.  Six LDS objects: the compiler
+// traffic), so every step issues the same 10.  Six LDS objects: the compiler
 // tells a direct-to-LDS load into one from reads of another.
 // ---------------------------------------------------------------------------
 constexpr int kI4TokBytes = kBM * 256;
-constexpr int kI4SxBytes = 8 * 512;  // per wave: 256 B scales (64 used), 256 B group sums
+constexpr int kI4SxBytes = 4 * 512;  // per wave: 256 B scales (128 used), 256 B group sums
 
 template <int PHASE, bool NARROW>
-__global__ void __launch_bounds__(512, 1) gemm2_i4_kernel(GemmArgs a, int n_slabs, int sg) {
-  constexpr int kWaves = 8;
-  constexpr int kRT = 2;
+__global__ void __launch_bounds__(256, 2) gemm2_i4_kernel(GemmArgs a, int n_slabs, int sg) {
+  constexpr int kWaves = 4;
+  constexpr int kRT = 4;
+  constexpr int kStepLoads = 10;  // a stage's loads per wave: 4 token, 4 weight, scales, group sums
   __shared__ __attribute__((aligned(1024))) uint8_t tb0[kI4TokBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t tb1[kI4TokBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t tb2[kI4TokBytes];
@@ -888,41 +897,47 @@ __global__ void __launch_bounds__(512, 1) gemm2_i4_kernel(GemmArgs a, int n_slab
 #pragma unroll
   for (int r = 0; r < kRT; ++r) {
     if (PHASE == PHASE_GATE_UP)
-      wrow[r] = (r == 0 ? 0 : a.I) + it.slab * 128 + wave * 16;
+      wrow[r] = (r < kRT / 2 ? 0 : a.I) + it.slab * 128 + wave * (128 / kWaves) + (r % (kRT / 2)) * 16;
     else
-      wrow[r] = it.slab * 256 + wave * 32 + r * 16;
-    wsrc[r] = (uint32_t)(wrow[r] >> 4) * (uint32_t)G * 1024u + lane * 16u;
+      wrow[r] = it.slab * 256 + wave * (256 / kWaves) + r * 16;
+    wsrc[r] = (uint32_t)(wrow[r] >> 4) * (uint32_t)G * 1024u;  // the same in every lane
   }
-  // scale lane (lanes 16-63 repeat lanes 0-15): row tile (l % 16) / 8, 4-byte piece l % 8
-  const int sl = lane & 15;
-  const uint32_t ssrc = ((uint32_t)(wrow[sl >> 3] >> 4) * (uint32_t)G * 16u) * 2u + (sl & 7) * 4u;
+  // scale lane (lanes 32-63 repeat lanes 0-31): row tile (l % 32) / 8, 4-byte piece l % 8
+  const int sl = (lane >> 3) & 3;
+  const int srow = sl == 0 ? wrow[0] : sl == 1 ? wrow[1] : sl == 2 ? wrow[2] : wrow[3];
+  const uint32_t ssrc = ((uint32_t)(srow >> 4) * (uint32_t)G * 16u) * 2u + (lane & 7) * 4u;
   const uint32_t xsrc = (uint32_t)srcl[lane] * (uint32_t)G * 4u;
-  uint32_t tsrc[2];
+  uint32_t tsrc[4];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int p = 8 * wave + 4 * j + (lane >> 4);
+  for (int j = 0; j < 4; ++j) {
+    const int p = 16 * wave + 4 * j + (lane >> 4);
     const int chunk = (lane & 15) ^ (p & 15);
     tsrc[j] = (uint32_t)srcl[p] * (uint32_t)a.K * 2u + chunk * 16u;
   }
-  const int tofs = wave * 2048;  // this wave's slice of a token buffer
+  const int tofs = wave * 4096;  // this wave's slice of a token buffer
   const int sofs = wave * 512;   // and of a scale / group-sum buffer
 
-  // stage st's 6 loads (st >= G: out of range, no traffic), the weights
-  // with the copy's load policy (tag >> 4: nt for an expert's only tile)
-  auto issue = [&](auto nc, int st, uint8_t* tb, uint8_t* sx, u32x4 (&w)[kRT]) {
+  // stage st's token, scale and group-sum loads, and its weight loads with
+  // the copy's load policy (tag >> 4: nt for an expert's only tile); st >= G:
+  // out of range, no traffic
+  auto issue_tok = [&](int st, uint8_t* tb, uint8_t* sx) __attribute__((always_inline)) {
+    const bool live = st < G;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(tres, (__attribute__((address_space(3))) void*)(tb + tofs + j * 1024),
+                                               16, live ? tsrc[j] : kI8Skip, live ? st * 256 : 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(sres, (__attribute__((address_space(3))) void*)(sx + sofs), 4,
+                                             live ? ssrc : kI8Skip, live ? st * 32 : 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (__attribute__((address_space(3))) void*)(sx + sofs + 256), 4,
+                                             live ? xsrc : kI8Skip, live ? st * 4 : 0, 0, 0);
+  };
+  auto issue_w = [&](auto nc, int st, u32x4 (&w)[kRT]) __attribute__((always_inline)) {
     constexpr int kPolicy = decltype(nc)::value >> 4;
     const bool live = st < G;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(tres, (__attribute__((address_space(3))) void*)(tb + tofs + j * 1024),
-                                               16, live ? tsrc[j] + st * 256u : kI8Skip, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(sres, (__attribute__((address_space(3))) void*)(sx + sofs), 4,
-                                             live ? ssrc + st * 32u : kI8Skip, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (__attribute__((address_space(3))) void*)(sx + sofs + 256), 4,
-                                             live ? xsrc + st * 4u : kI8Skip, 0, 0, 0);
-#pragma unroll
     for (int r = 0; r < kRT; ++r)
-      w[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wres, live ? wsrc[r] + st * 1024u : kI8Skip, 0, kPolicy));
+      w[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wres, live ? lane * 16u : kI8Skip,
+                                                                             live ? wsrc[r] + st * 1024u : 0u, kPolicy));
   };
 
   f32x4 acc[kRT][kCT];
@@ -931,72 +946,83 @@ __global__ void __launch_bounds__(512, 1) gemm2_i4_kernel(GemmArgs a, int n_slab
 #pragma unroll
     for (int c = 0; c < kCT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // all (row tile, column tile) temporaries advance one K step at a time,
-  // so no MFMA waits on the one before it; only the first NC column tiles
-  auto compute = [&](auto nc, const u32x4 (&w)[kRT], const uint8_t* tb, const uint8_t* sx) {
+  // one column tile at a time: its 4 row tiles' temporaries advance one K
+  // step at a time (4 independent chains; the CU's second workgroup fills
+  // what they leave), then the group scales; only the first NC column tiles
+  auto compute = [&](auto nc, const u32x4 (&ad)[kRT][4], const uint8_t* tb, const uint8_t* sx) __attribute__((always_inline)) {
     constexpr int NC = decltype(nc)::value & 15;
-    u32x4 bf[kCT][4];
+    f32x4 sc[kRT];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
+    for (int r = 0; r < kRT; ++r) sc[r] = bf16x4_to_f32(*(const u32x2*)(sx + sofs + r * 32 + (lane >> 4) * 8));
+    u32x4 bf[2][4];
+    auto read_b = [&](u32x4 (&f)[4], int c) __attribute__((always_inline)) {
       const int p = c * 16 + (lane & 15);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) bf[c][s] = *(const u32x4*)(tb + p * 256 + (((4 * s + (lane >> 4)) ^ (p & 15)) * 16));
-    }
-    u32x4 ad[kRT][4];
-    f32x4 sc[kRT];
-    const DqConst kdq = dq_const();
-#pragma unroll
-    for (int r = 0; r < kRT; ++r) {
-      sc[r] = bf16x4_to_f32(*(const u32x2*)(sx + sofs + r * 32 + (lane >> 4) * 8));
-#pragma unroll
-      for (int s = 0; s < 4; ++s) ad[r][s] = dq_i4_k(w[r][s], kdq);
-    }
-    f32x4 tmp[kRT][kCT];
+      for (int s = 0; s < 4; ++s) f[s] = *(const u32x4*)(tb + p * 256 + (((4 * s + (lane >> 4)) ^ (p & 15)) * 16));
+    };
+    read_b(bf[0], 0);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
+      if (c + 1 < NC) read_b(bf[(c + 1) & 1], c + 1);
       const float cv = -136.0f * *(const float*)(sx + sofs + 256 + (c * 16 + (lane & 15)) * 4);
+      f32x4 tmp[kRT];
 #pragma unroll
-      for (int r = 0; r < kRT; ++r) tmp[r][c] = f32x4{cv, cv, cv, cv};
+      for (int r = 0; r < kRT; ++r) tmp[r] = f32x4{cv, cv, cv, cv};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int r = 0; r < kRT; ++r) tmp[r] = mfma_bf16(ad[r][s], bf[c & 1][s], tmp[r]);
+#pragma unroll
+      for (int r = 0; r < kRT; ++r) acc[r][c] += sc[r] * tmp[r];
+      __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int r = 0; r < kRT; ++r) tmp[r][c] = mfma_bf16(ad[r][s], bf[c][s], tmp[r][c]);
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int r = 0; r < kRT; ++r) acc[r][c] += sc[r] * tmp[r][c];
   };
 
-  u32x4 w0[kRT], w1[kRT], w2[kRT];
-  auto step = [&](auto nc, const u32x4 (&wcur)[kRT], u32x4 (&wn2)[kRT], const uint8_t* tb_x, const uint8_t* sx_x,
-                  uint8_t* tb_n2, uint8_t* sx_n2, int x) {
-    __asm__ volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0F76);  // vmcnt(6): stage x landed (stage x + 1's 6 may fly)
+  u32x4 w0[kRT], w1[kRT];
+  // a stage's weights are dequantised first, which frees their registers for
+  // the loads of two stages on (a ring of two)
+  auto step = [&](auto nc, u32x4 (&w)[kRT], const uint8_t* tb_x, const uint8_t* sx_x, uint8_t* tb_n2,
+                  uint8_t* sx_n2, int x) __attribute__((always_inline)) {
+    wait_vmem_but<kStepLoads>();  // stage x landed (stage x + 1's loads may fly)
     lds_barrier();
-    issue(nc, x + 2, tb_n2, sx_n2, wn2);
-    compute(nc, wcur, tb_x, sx_x);
+    issue_tok(x + 2, tb_n2, sx_n2);
+    u32x4 ad[kRT][4];
+    const DqConst kdq = dq_const();
+#pragma unroll
+    for (int r = 0; r < kRT; ++r)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) ad[r][s] = dq_i4_k(w[r][s], kdq);
+    issue_w(nc, x + 2, w);
+    compute(nc, ad, tb_x, sx_x);
     __builtin_amdgcn_sched_barrier(0);
   };
   // the pipeline over the first NC column tiles, one copy per NC
-  auto run = [&](auto nc) {
-    issue(nc, 0, tb0, sx0, w0);
-    issue(nc, 1, tb1, sx1, w1);
-    // three steps per iteration return ring slots and buffers to their roles
+  auto run = [&](auto nc) __attribute__((always_inline)) {
+    issue_tok(0, tb0, sx0);
+    issue_w(nc, 0, w0);
+    issue_tok(1, tb1, sx1);
+    issue_w(nc, 1, w1);
+    // six steps per iteration return registers and buffers to their roles
     int x = 0;
-    for (; x + 3 <= G; x += 3) {
-      step(nc, w0, w2, tb0, sx0, tb2, sx2, x);
-      step(nc, w1, w0, tb1, sx1, tb0, sx0, x + 1);
-      step(nc, w2, w1, tb2, sx2, tb1, sx1, x + 2);
+    for (; x + 6 <= G; x += 6) {
+      step(nc, w0, tb0, sx0, tb2, sx2, x);
+      step(nc, w1, tb1, sx1, tb0, sx0, x + 1);
+      step(nc, w0, tb2, sx2, tb1, sx1, x + 2);
+      step(nc, w1, tb0, sx0, tb2, sx2, x + 3);
+      step(nc, w0, tb1, sx1, tb0, sx0, x + 4);
+      step(nc, w1, tb2, sx2, tb1, sx1, x + 5);
     }
-    if (x < G) step(nc, w0, w2, tb0, sx0, tb2, sx2, x);
-    if (x + 1 < G) step(nc, w1, w0, tb1, sx1, tb0, sx0, x + 1);
+    const int rest = G - x;
+    if (rest >= 1) step(nc, w0, tb0, sx0, tb2, sx2, x);
+    if (rest >= 2) step(nc, w1, tb1, sx1, tb0, sx0, x + 1);
+    if (rest >= 3) step(nc, w0, tb2, sx2, tb1, sx1, x + 2);
+    if (rest >= 4) step(nc, w1, tb0, sx0, tb2, sx2, x + 3);
+    if (rest >= 5) step(nc, w0, tb1, sx1, tb0, sx0, x + 4);
     wait_vmem();  // out-of-range loads past the last stage land before the LDS is reused
     __syncthreads();
+    // down's compact y staging: 16 rows of 144 B per wave in a token buffer
     gemm2_epilogue<WF_I4, PHASE, kWaves>(a, acc, srcl, orow_l, hpart, xtot_l, xtot_l, wrow, sexp, it.row0, it.rows,
-                                         it.slab);
+                                         it.slab, nullptr, PHASE == PHASE_DOWN ? tb0 + wave * 2304 : nullptr);
   };
   // NARROW (experts average at most 48 positions): a tile of at most 16 / 32
   // / 48 positions, an expert's last or only one, runs 1 / 2 / 3 of its 4
@@ -1035,23 +1061,7 @@ __global__ void __launch_bounds__(512, 1) gemm2_i4_kernel(GemmArgs a, int n_slab
       run(std::integral_constant<int, kCT>{});
     }
   } else {
-    // (the same pipeline written out: a launch of full tiles keeps the
-    // schedule the compiler gives it without the lambda, 1 - 2 % faster)
-    const std::integral_constant<int, kCT> nc;
-    issue(nc, 0, tb0, sx0, w0);
-    issue(nc, 1, tb1, sx1, w1);
-    int x = 0;
-    for (; x + 3 <= G; x += 3) {
-      step(nc, w0, w2, tb0, sx0, tb2, sx2, x);
-      step(nc, w1, w0, tb1, sx1, tb0, sx0, x + 1);
-      step(nc, w2, w1, tb2, sx2, tb1, sx1, x + 2);
-    }
-    if (x < G) step(nc, w0, w2, tb0, sx0, tb2, sx2, x);
-    if (x + 1 < G) step(nc, w1, w0, tb1, sx1, tb0, sx0, x + 1);
-    wait_vmem();
-    __syncthreads();
-    gemm2_epilogue<WF_I4, PHASE, kWaves>(a, acc, srcl, orow_l, hpart, xtot_l, xtot_l, wrow, sexp, it.row0, it.rows,
-                                         it.slab);
+    run(std::integral_constant<int, kCT>{});
   }
 }
 
@@ -1249,6 +1259,7 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
     return hipGetLastError();
   }
   if (gemm2_i4_pipeline(a, wf)) {
+    block = dim3(256);
     if (phase == PHASE_GATE_UP && a.narrow_tiles)
       launch_timed(gemm2_i4_kernel<PHASE_GATE_UP, true>, grid, block, 0, stream, tm, a, n_slabs, sg);
     else if (phase == PHASE_GATE_UP)

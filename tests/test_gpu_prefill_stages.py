@@ -1,0 +1,31 @@
+"""Prefill-form expert GEMMs at the edges of their K pipelines and token tiles.
+
+Two experts that every token picks, so each holds T positions: T around the
+16-position column tiles and the 64-position tiles, and H / I so that gate_up
+and down end in every remainder of the unrolled stage loop (1 .. 8 stages of
+128).  Tolerance as in moe_cases.compare (bf16 outputs)."""
+from dataclasses import replace
+
+import pytest
+import torch
+
+from moe_cases import CONFIGS, build_inputs, build_layer, compare, native_layer, oracle_forward
+
+pytestmark = pytest.mark.gpu
+
+# (H, I): gate_up runs H / 128 stages, down I / 128
+SHAPES = [(256, 128), (512, 384), (768, 640), (1024, 256), (1280, 896), (256, 512)]
+
+
+@pytest.mark.parametrize("wfmt", ["int4_g128"])
+@pytest.mark.parametrize("H,I", SHAPES)
+def test_stage_and_tile_remainders(gpu_device, wfmt, H, I):
+    cfg = replace(CONFIGS["qwen3_int4"], name=f"stages_{wfmt}", H=H, I=I, E=2, k=2, wfmt=wfmt)
+    layer = build_layer(cfg, device="cuda")
+    native = native_layer(layer, torch.device("cuda"))
+    for T in (13, 17, 33, 49, 64, 65, 130):
+        x, logits = build_inputs(layer, T, seed=T, device="cuda")
+        out = native.forward(x, logits)
+        torch.cuda.synchronize()
+        ref = oracle_forward(layer, x, logits)
+        compare(out.float().cpu().numpy(), ref, cfg)
