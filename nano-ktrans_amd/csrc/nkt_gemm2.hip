@@ -852,6 +852,9 @@ bool gemm2_supported(int wf, int phase, int N, int K, int I) {
 // waves -> this: Mixtral T = 2048 gate_up 1081 -> 933 us (890 -> 1031
 // TFLOP/s), down 588 -> 536; Qwen3 T = 2048 gate_up 185 -> 164, down 124 ->
 // 96; Qwen3 T = 203 (narrow copies) gate_up 47.7 -> 44.4, down 33.4 -> 27.1.
+// KS = 2 (launch_gemm2's rule): eight waves, the second four on the second
+// half of K with buffers of their own, for launches too small to give every
+// CU two workgroups.
 // Loads past the last stage take an out-of-range buffer offset (no
 // traffic), so every step issues the same 10.  Six LDS objects: the compiler
 // tells a direct-to-LDS load into one from reads of another.
@@ -859,17 +862,17 @@ bool gemm2_supported(int wf, int phase, int N, int K, int I) {
 constexpr int kI4TokBytes = kBM * 256;
 constexpr int kI4SxBytes = 4 * 512;  // per wave: 256 B scales (128 used), 256 B group sums
 
-template <int PHASE, bool NARROW>
-__global__ void __launch_bounds__(256, 2) gemm2_i4_kernel(GemmArgs a, int n_slabs, int sg) {
+template <int PHASE, bool NARROW, int KS = 1>
+__global__ void __launch_bounds__(256 * KS, 2) gemm2_i4_kernel(GemmArgs a, int n_slabs, int sg) {
   constexpr int kWaves = 4;
   constexpr int kRT = 4;
   constexpr int kStepLoads = 10;  // a stage's loads per wave: 4 token, 4 weight, scales, group sums
-  __shared__ __attribute__((aligned(1024))) uint8_t tb0[kI4TokBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t tb1[kI4TokBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t tb2[kI4TokBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t sx0[kI4SxBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t sx1[kI4SxBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t sx2[kI4SxBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t tb0[KS * kI4TokBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t tb1[KS * kI4TokBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t tb2[KS * kI4TokBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t sx0[KS * kI4SxBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t sx1[KS * kI4SxBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t sx2[KS * kI4SxBytes];
   __shared__ int srcl[kBM];
   __shared__ int orow_l[kBM];
   __shared__ float hpart[kWaves][kBM];
@@ -878,19 +881,22 @@ __global__ void __launch_bounds__(256, 2) gemm2_i4_kernel(GemmArgs a, int n_slab
   TileItem it;
   if (!gemm2_item(a, n_slabs, sg, it)) return;
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % kWaves;
+  const int part = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;  // this wave's K part
   gemm2_sources(a, it, srcl, orow_l);
   __syncthreads();
 
   const uint16_t* sexp = a.scales + (int64_t)it.expert * a.s_expert_elems;
-  const int G = a.K / 128;  // stages = scale groups = 1 KiB blocks per 16-row block
+  const int Grow = a.K / 128;  // scale groups = 1 KiB blocks per 16-row block
+  const int G = Grow / KS;     // stages of this wave's K part
+  const int g0 = part * G;
   const int rows_in = (int)(a.in_bytes / ((int64_t)a.K * 2));
   const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(a.w + (int64_t)it.expert * a.w_expert_bytes), (short)0, (int)a.w_expert_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t sres =
       __builtin_amdgcn_make_buffer_rsrc((void*)sexp, (short)0, (int)(a.s_expert_elems * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t xres =
-      __builtin_amdgcn_make_buffer_rsrc((void*)a.xsum, (short)0, rows_in * G * 4, 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.xsum, (short)0, rows_in * Grow * 4, 0x00020000);
   const __amdgpu_buffer_rsrc_t tres = __builtin_amdgcn_make_buffer_rsrc((void*)a.in, (short)0, (int)a.in_bytes, 0x00020000);
   int wrow[kRT];
   uint32_t wsrc[kRT];
@@ -900,22 +906,23 @@ __global__ void __launch_bounds__(256, 2) gemm2_i4_kernel(GemmArgs a, int n_slab
       wrow[r] = (r < kRT / 2 ? 0 : a.I) + it.slab * 128 + wave * (128 / kWaves) + (r % (kRT / 2)) * 16;
     else
       wrow[r] = it.slab * 256 + wave * (256 / kWaves) + r * 16;
-    wsrc[r] = (uint32_t)(wrow[r] >> 4) * (uint32_t)G * 1024u;  // the same in every lane
+    wsrc[r] = ((uint32_t)(wrow[r] >> 4) * (uint32_t)Grow + (uint32_t)g0) * 1024u;  // the same in every lane
   }
   // scale lane (lanes 32-63 repeat lanes 0-31): row tile (l % 32) / 8, 4-byte piece l % 8
   const int sl = (lane >> 3) & 3;
   const int srow = sl == 0 ? wrow[0] : sl == 1 ? wrow[1] : sl == 2 ? wrow[2] : wrow[3];
-  const uint32_t ssrc = ((uint32_t)(srow >> 4) * (uint32_t)G * 16u) * 2u + (lane & 7) * 4u;
-  const uint32_t xsrc = (uint32_t)srcl[lane] * (uint32_t)G * 4u;
+  const uint32_t ssrc = ((uint32_t)(srow >> 4) * (uint32_t)Grow + (uint32_t)g0) * 32u + (lane & 7) * 4u;
+  const uint32_t xsrc = ((uint32_t)srcl[lane] * (uint32_t)Grow + (uint32_t)g0) * 4u;
   uint32_t tsrc[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int p = 16 * wave + 4 * j + (lane >> 4);
     const int chunk = (lane & 15) ^ (p & 15);
-    tsrc[j] = (uint32_t)srcl[p] * (uint32_t)a.K * 2u + chunk * 16u;
+    tsrc[j] = (uint32_t)srcl[p] * (uint32_t)a.K * 2u + (uint32_t)g0 * 256u + chunk * 16u;
   }
-  const int tofs = wave * 4096;  // this wave's slice of a token buffer
-  const int sofs = wave * 512;   // and of a scale / group-sum buffer
+  const int tpart = part * kI4TokBytes;                // this K part's token buffer
+  const int tofs = tpart + wave * 4096;                // this wave's slice of it
+  const int sofs = part * kI4SxBytes + wave * 512;     // and of a scale / group-sum buffer
 
   // stage st's token, scale and group-sum loads, and its weight loads with
   // the copy's load policy (tag >> 4: nt for an expert's only tile); st >= G:
@@ -958,7 +965,7 @@ __global__ void __launch_bounds__(256, 2) gemm2_i4_kernel(GemmArgs a, int n_slab
     auto read_b = [&](u32x4 (&f)[4], int c) __attribute__((always_inline)) {
       const int p = c * 16 + (lane & 15);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) f[s] = *(const u32x4*)(tb + p * 256 + (((4 * s + (lane >> 4)) ^ (p & 15)) * 16));
+      for (int s = 0; s < 4; ++s) f[s] = *(const u32x4*)(tb + tpart + p * 256 + (((4 * s + (lane >> 4)) ^ (p & 15)) * 16));
     };
     read_b(bf[0], 0);
 #pragma unroll
@@ -1020,9 +1027,28 @@ __global__ void __launch_bounds__(256, 2) gemm2_i4_kernel(GemmArgs a, int n_slab
     if (rest >= 5) step(nc, w0, tb1, sx1, tb0, sx0, x + 4);
     wait_vmem();  // out-of-range loads past the last stage land before the LDS is reused
     __syncthreads();
+    if constexpr (KS > 1) {
+      // the second K part's sums reach the first through the token buffers
+      // (16 bytes per lane, one 1 KiB row per wave and tile); its waves end
+      auto slot = [&](int r, int c) __attribute__((always_inline)) {
+        return (f32x4*)((r < 2 ? tb0 : tb1) + (((r & 1) * kCT + c) * kWaves + wave) * 1024 + lane * 16);
+      };
+      if (part == 1) {
+#pragma unroll
+        for (int r = 0; r < kRT; ++r)
+#pragma unroll
+          for (int c = 0; c < kCT; ++c) *slot(r, c) = acc[r][c];
+      }
+      __syncthreads();
+      if (part == 1) return;
+#pragma unroll
+      for (int r = 0; r < kRT; ++r)
+#pragma unroll
+        for (int c = 0; c < kCT; ++c) acc[r][c] += *slot(r, c);
+    }
     // down's compact y staging: 16 rows of 144 B per wave in a token buffer
     gemm2_epilogue<WF_I4, PHASE, kWaves>(a, acc, srcl, orow_l, hpart, xtot_l, xtot_l, wrow, sexp, it.row0, it.rows,
-                                         it.slab, nullptr, PHASE == PHASE_DOWN ? tb0 + wave * 2304 : nullptr);
+                                         it.slab, nullptr, PHASE == PHASE_DOWN ? tb2 + wave * 2304 : nullptr);
   };
   // NARROW (experts average at most 48 positions): a tile of at most 16 / 32
   // / 48 positions, an expert's last or only one, runs 1 / 2 / 3 of its 4
@@ -1230,6 +1256,16 @@ hipError_t launch_group_sums(const void* x, int rows, int K, float* out, hipStre
 // int4 adds per-group scale temporaries) and removes their spills.
 constexpr int gemm2_waves(int wf) { return wf == WF_I8 ? 4 : 8; }
 
+// The int4 down runs its K in two halves on eight waves (KS = 2) while the
+// launch has at most this many (token tile, weight slab) items (counted with
+// the tile list's upper bound): one workgroup per CU or fewer, so two
+// four-wave workgroups never share a CU and the long K loop (Mixtral: 112
+// stages on 16 slabs x 8 experts = 128 items) is the whole launch.  Measured,
+// Mixtral-8x7B int4, one part -> two, us per layer: T = 100 209 -> 190; eight
+// waves of 32 rows on all of K (before): T = 40 / 100 / 180 178 / 204 / 262
+// -> 167 / 190 / 241, T = 240 (the rule's edge) 324 -> 322.
+constexpr int64_t kI4SplitMaxItems = 256;
+
 hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hipStream_t stream,
                         const KernelTimer* tm) {
   if (max_tiles <= 0) return hipSuccess;
@@ -1264,6 +1300,8 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
       launch_timed(gemm2_i4_kernel<PHASE_GATE_UP, true>, grid, block, 0, stream, tm, a, n_slabs, sg);
     else if (phase == PHASE_GATE_UP)
       launch_timed(gemm2_i4_kernel<PHASE_GATE_UP, false>, grid, block, 0, stream, tm, a, n_slabs, sg);
+    else if (a.narrow_tiles && items <= kI4SplitMaxItems && a.K % 256 == 0)
+      launch_timed(gemm2_i4_kernel<PHASE_DOWN, true, 2>, grid, dim3(512), 0, stream, tm, a, n_slabs, sg);
     else if (a.narrow_tiles)
       launch_timed(gemm2_i4_kernel<PHASE_DOWN, true>, grid, block, 0, stream, tm, a, n_slabs, sg);
     else
