@@ -6,16 +6,18 @@
 // PackedSparseExpertMLP.forward, nano_ktrans/layers/expert_mlp.py:20-41) and
 // the quantized loop of nano_ktrans/kernels/cpu_moe.py:419-450.
 //
-// Three kernels share the work order, tile record and epilogue:
+// Four kernels share the work order, tile record and epilogue:
 //   * gemm2_i8_kernel (int8): 4 waves, three-stage pipeline of 64-wide K
 //     stages (tokens direct-to-LDS, weights in a register ring), gate_up on
 //     the fp16 matrix cores;
 //   * gemm2_i4_kernel (int4 g128): 4 waves, three-stage pipeline of 128-wide
 //     K stages (tokens, scales and group sums direct-to-LDS, weights in a
 //     ring of two register stages);
-//   * gemm2_kernel (bf16 weights, and int8 / int4 operands past the
-//     pipelines' 32-bit buffer offsets): the register-staged form below.
-// The two pipelines also hold copies that compute only the first 16 / 32
+//   * gemm2_bf16_kernel (bf16): the int8 pipeline's form, two weight blocks
+//     per row tile and stage;
+//   * gemm2_kernel (operands past the pipelines' 32-bit buffer offsets): the
+//     register-staged form below.
+// The pipelines also hold copies that compute only the first 16 / 32
 // positions of a tile, taken by tiles with no more (an expert's last or
 // only tile): the matrix-core work of empty column tiles is skipped, and an
 // expert's only tile loads its weights non-temporally.
@@ -539,7 +541,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) gemm2_kernel(GemmArgs a, int n
 }
 
 // ---------------------------------------------------------------------------
-// int8 weights, three-stage pipeline.  Same tile, waves, work order, MFMA
+// int8 (and bf16) weights, three-stage pipeline.  Same tile, waves, work order, MFMA
 // sequence and epilogue as gemm2_kernel<WF_I8, ...> (so the results are the
 // same bit for bit); K advances in 64-wide stages:
 //   * weights: each wave's own 4 row tiles, one 1 KiB block (16 rows x 64 K,
@@ -566,10 +568,16 @@ constexpr int kI8Stage = 64;                   // K per stage
 constexpr int kI8TokBytes = kBM * kI8Stage * 2;
 constexpr uint32_t kI8Skip = 0xFFFFFF00u;     // a buffer offset past every range the kernel is given
 
-template <int PHASE, bool F16>
-__global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slabs, int sg) {
+// bf16 weights: an offset past every range that stays past it, without
+// wrapping, when a row offset below it is added
+constexpr uint32_t kBf16Skip = 0x80000000u;
+
+template <int WF, int PHASE, bool F16>
+__device__ __forceinline__ void gemm2_stage64(const GemmArgs& a, int n_slabs, int sg) {
   constexpr int kWaves = 4;
   constexpr int kRT = 4;
+  constexpr int NB = kI8Stage / block_k(WF);  // 1 KiB weight blocks per row tile and stage: int8 1, bf16 2
+  constexpr int kStepLoads = 2 + kRT * NB;    // a stage's loads per wave
   __shared__ __attribute__((aligned(1024))) uint8_t tb0[kI8TokBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t tb1[kI8TokBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t tb2[kI8TokBytes];
@@ -595,11 +603,11 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
   const int Kp = (PHASE == PHASE_DOWN && a.k_parts > 1) ? a.K / a.k_parts : a.K;  // this item's K range
   const uint16_t* sexp = a.scales + (int64_t)it.expert * a.s_expert_elems;
   const int NS = Kp / kI8Stage;         // stages this item runs
-  const int NSrow = a.K / kI8Stage;     // 1 KiB blocks per 16-row block
+  const int NSrow = a.K / kI8Stage * NB;  // 1 KiB blocks per 16-row block
   // buffer resources over this expert's weights and the activation rows; a
   // load at offset kI8Skip is out of range: it reads nothing (zeros)
   const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(a.w + (int64_t)it.expert * a.w_expert_bytes), (short)0, a.N * a.K, 0x00020000);
+      (void*)(a.w + (int64_t)it.expert * a.w_expert_bytes), (short)0, (int)a.w_expert_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t tres = __builtin_amdgcn_make_buffer_rsrc((void*)a.in, (short)0, a.in_bytes, 0x00020000);
   int wrow[kRT];
   uint32_t wsrc[kRT];
@@ -609,7 +617,8 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
       wrow[r] = (r < kRT / 2 ? 0 : a.I) + it.slab * 128 + wave * (128 / kWaves) + (r % (kRT / 2)) * 16;
     else
       wrow[r] = it.slab * 256 + wave * (256 / kWaves) + r * 16;
-    wsrc[r] = ((uint32_t)(wrow[r] >> 4) * (uint32_t)NSrow + (uint32_t)(kpart * NS)) * 1024u + lane * 16u;
+    wsrc[r] = ((uint32_t)(wrow[r] >> 4) * (uint32_t)NSrow + (uint32_t)(kpart * NS * NB)) * 1024u +
+              (WF == WF_I8 ? lane * 16u : 0u);
   }
   uint32_t tsrc[2];
 #pragma unroll
@@ -628,14 +637,20 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
       __builtin_amdgcn_raw_ptr_buffer_load_lds(tres, (__attribute__((address_space(3))) void*)(tb + tofs + j * 1024),
                                                16, live ? tsrc[j] + st * (kI8Stage * 2u) : kI8Skip, 0, 0, 0);
   };
-  // stage st's 4 weight blocks into registers, with the copy's load policy
+  // stage st's weight blocks into registers, with the copy's load policy
   // (nt for an expert's only tile: no other item reads its weights)
-  auto issue_w = [&](auto nc, int st, u32x4 (&w)[kRT]) {
+  typedef u32x4 WRegs[kRT][NB];
+  auto issue_w = [&](auto nc, int st, WRegs& w) {
     constexpr int kPolicy = decltype(nc)::value >> 4;
     const bool live = st < NS;
 #pragma unroll
     for (int r = 0; r < kRT; ++r)
-      w[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wres, live ? wsrc[r] + st * 1024u : kI8Skip, 0, kPolicy));
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+        w[r][i] = __builtin_bit_cast(
+            u32x4, WF == WF_I8 ? __builtin_amdgcn_raw_buffer_load_b128(wres, live ? wsrc[r] + st * 1024u : kI8Skip, 0, kPolicy)
+                               : __builtin_amdgcn_raw_buffer_load_b128(
+                                     wres, (live ? lane * 16u + st * (NB * 1024u) : kBf16Skip) + i * 1024u, wsrc[r], kPolicy));
   };
 
   f32x4 acc[kRT][kCT];
@@ -660,13 +675,18 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
         f[s][c] = *(const u32x4*)(tb + p * (kI8Stage * 2) + ((chunk ^ ((p >> 1) & 7)) * 16));
       }
   };
-  auto mma = [&](auto nc, const u32x4 (&w)[kRT], const TokFrags& f) {
+  auto mma = [&](auto nc, const WRegs& w, const TokFrags& f) {
     constexpr int NC = decltype(nc)::value & 15;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       u32x4 ad[kRT];
 #pragma unroll
-      for (int r = 0; r < kRT; ++r) ad[r] = F16 ? dq_i8_f16(w[r][2 * s], w[r][2 * s + 1]) : dq_i8(w[r][2 * s], w[r][2 * s + 1]);
+      for (int r = 0; r < kRT; ++r) {
+        if constexpr (WF == WF_BF16)
+          ad[r] = w[r][s];
+        else
+          ad[r] = F16 ? dq_i8_f16(w[r][0][2 * s], w[r][0][2 * s + 1]) : dq_i8(w[r][0][2 * s], w[r][0][2 * s + 1]);
+      }
 #pragma unroll
       for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -676,14 +696,13 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
   };
 
   TokFrags f0, f1;
-  u32x4 w0[kRT], w1[kRT], w2[kRT];
+  WRegs w0, w1, w2;
   // issue order: T0, T1, W0, T2, W1, then per step x: T(x + 3), W(x + 2);
-  // at step x the newest 6 loads are T(x + 2) and W(x + 1), so waiting for
-  // all but 6 covers T(x + 1) and W(x)
-  auto step = [&](auto nc, TokFrags& cur, TokFrags& nxt, const u32x4 (&wcur)[kRT], u32x4 (&wnew)[kRT],
-                  uint8_t* tb_x, const uint8_t* tb_n, int x) {
-    __asm__ volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0F76);  // vmcnt(6)
+  // at step x the newest loads are T(x + 2) and W(x + 1), so waiting for
+  // all but those covers T(x + 1) and W(x)
+  auto step = [&](auto nc, TokFrags& cur, TokFrags& nxt, const WRegs& wcur, WRegs& wnew, uint8_t* tb_x,
+                  const uint8_t* tb_n, int x) {
+    wait_vmem_but<kStepLoads>();
     lds_barrier();
     issue_tok(x + 3, tb_x);
     issue_w(nc, x + 2, wnew);
@@ -701,7 +720,7 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
   auto run = [&](auto nc) {
     EpiPre<kRT> pre;
     float rv[16], rxi = 0.f;
-    pre.valid = i8_row_terms<F16>(a, srcl, rv, rxi, kpart * (Kp / 128), Kp / 128);
+    pre.valid = WF == WF_I8 && i8_row_terms<F16>(a, srcl, rv, rxi, kpart * (Kp / 128), Kp / 128);
     if (pre.valid) {
 #pragma unroll
       for (int r = 0; r < kRT; ++r) pre.s[r] = *(const u32x2*)(sexp + wrow[r] + 4 * (lane >> 4));
@@ -712,8 +731,7 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
     issue_tok(2, tb2);
     issue_w(nc, 1, w1);
     if (pre.valid) i8_row_terms_store(Kp / 128, xtot_l, xinv_l, rv, rxi, F16);
-    __asm__ volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0F7C);  // vmcnt(12): T0 landed
+    wait_vmem_but<2 * kStepLoads>();  // T0 landed
     lds_barrier();
     read_tok(nc, f0, tb0);
     // six steps per iteration return fragments, weight registers and buffers
@@ -738,7 +756,7 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
     // down's compact y staging: 16 rows of 144 B per wave in the token
     // buffers, free once every wave has passed the barrier above
     uint8_t* stage = wave < 3 ? tb0 + wave * 2304 : tb1;
-    gemm2_epilogue<WF_I8, PHASE, kWaves, F16>(a, acc, srcl, orow_l, hpart, xtot_l, xinv_l, wrow, sexp, it.row0, it.rows,
+    gemm2_epilogue<WF, PHASE, kWaves, F16>(a, acc, srcl, orow_l, hpart, xtot_l, xinv_l, wrow, sexp, it.row0, it.rows,
                                               it.slab, &pre, PHASE == PHASE_DOWN ? stage : nullptr,
                                               (int64_t)kpart * a.num_rows * a.N);
   };
@@ -769,8 +787,31 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
     else
       run(std::integral_constant<int, 3>{});
   } else {
-    run(std::integral_constant<int, kCT>{});
+    if (WF == WF_BF16 && only)
+      run(std::integral_constant<int, kCT | 2 << 4>{});
+    else
+      run(std::integral_constant<int, kCT>{});
   }
+}
+
+template <int PHASE, bool F16>
+__global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slabs, int sg) {
+  gemm2_stage64<WF_I8, PHASE, F16>(a, n_slabs, sg);
+}
+
+// bf16 weights on the same pipeline: two 1 KiB blocks per row tile and stage
+// (32 columns each), no dequantisation, the weights' row offsets in scalar
+// registers (one vector offset serves all eight loads; with a vector offset
+// per row the nt copy of the full tile spilled).  Bound by the weight stream
+// from HBM until experts hold a few tiles, then by waits; the register-staged
+// gemm2_kernel kept one eight-wave workgroup per CU and no short-tile copies.
+// Measured, gemm2_kernel -> this (Qwen3 bf16, us per layer): T = 200 / 700 /
+// 1000 / 2000 / 4096 230 / 275 / 282 / 375 / 606 -> 207 / 249 / 277 / 356 /
+// 535; the full tile's nt copy (an expert's only tile of 49 - 64 positions)
+// T = 850 / 1000 265 / 285 -> 250 / 277.
+template <int PHASE>
+__global__ void __launch_bounds__(256, 2) gemm2_bf16_kernel(GemmArgs a, int n_slabs, int sg) {
+  gemm2_stage64<WF_BF16, PHASE, false>(a, n_slabs, sg);
 }
 
 // Per-row sums of each 128-wide K group of a bf16 matrix [rows, K] -> fp32
@@ -805,6 +846,11 @@ __global__ void __launch_bounds__(256) group_sums_kernel(const uint16_t* __restr
 // the int8 pipeline addresses its operands with 32-bit buffer offsets
 bool gemm2_i8_pipeline(const GemmArgs& a, int wf) {
   return wf == WF_I8 && a.in_bytes <= (int64_t)kI8Skip && (int64_t)a.N * a.K <= (int64_t)kI8Skip;
+}
+
+// the same for bf16 weights (bf16 activations)
+bool gemm2_bf16_pipeline(const GemmArgs& a, int wf) {
+  return wf == WF_BF16 && a.in_bytes > 0 && a.in_bytes <= (int64_t)kI8Skip && a.w_expert_bytes < (int64_t)kBf16Skip;
 }
 
 // the int4 pipeline addresses weights, scales, group sums and activations
@@ -1292,6 +1338,13 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
       launch_timed(gemm2_i8_kernel<PHASE_GATE_UP, false>, grid, block, 0, stream, tm, a, n_slabs, sg);
     else
       launch_timed(gemm2_i8_kernel<PHASE_DOWN, false>, grid, block, 0, stream, tm, a, n_slabs, sg);
+    return hipGetLastError();
+  }
+  if (gemm2_bf16_pipeline(a, wf)) {
+    if (phase == PHASE_GATE_UP)
+      launch_timed(gemm2_bf16_kernel<PHASE_GATE_UP>, grid, dim3(256), 0, stream, tm, a, n_slabs, sg);
+    else
+      launch_timed(gemm2_bf16_kernel<PHASE_DOWN>, grid, dim3(256), 0, stream, tm, a, n_slabs, sg);
     return hipGetLastError();
   }
   if (gemm2_i4_pipeline(a, wf)) {

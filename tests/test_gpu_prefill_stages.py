@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(256, 128), (512, 384), (768, 640), (1024, 256), (1280, 896), (256, 512)]
 
 
-@pytest.mark.parametrize("wfmt", ["int4_g128"])
+@pytest.mark.parametrize("wfmt", ["int4_g128", "bf16", "int8_per_channel"])
 @pytest.mark.parametrize("H,I", SHAPES)
 def test_stage_and_tile_remainders(gpu_device, wfmt, H, I):
     cfg = replace(CONFIGS["qwen3_int4"], name=f"stages_{wfmt}", H=H, I=I, E=2, k=2, wfmt=wfmt)
