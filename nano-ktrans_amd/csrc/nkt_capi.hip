@@ -361,9 +361,10 @@ GemmArgs expert_args(const Handle* h, int phase, bool shared, const void* in, vo
 
 constexpr int kSpreadMinTokens = 16;
 
-// prep (nullable): the int8 gate_up's fp16 input to make in the routing
+// prep (nullable): the input of the prefill gate_up to prepare in the routing
 // launch when routing takes the large-batch path (*prep_done says whether it
-// did); prep_first: take that path for any T (a shared expert then forks
+// did): int8's fp16 copy (prep->in16 set) with its group sums, or int4's
+// group sums; prep_first: take that path for any T (a shared expert then forks
 // beside the routed experts as soon as the copy exists)
 int do_route(Handle* h, const void* logits, int T, void* ws, const WsLayout& L, hipStream_t st,
              char* err, size_t len, const GemmArgs* prep = nullptr, bool* prep_done = nullptr,
@@ -403,7 +404,13 @@ int do_route(Handle* h, const void* logits, int T, void* ws, const WsLayout& L, 
       return NKT_ERR;
     return NKT_OK;
   }
-  if (prep && h->act_bf16) {
+  if (prep && h->act_bf16 && !prep->in16) {
+    if (!check_hip(launch_route_sums(logits, T, h->E, h->k, h->flags, ids, wts, prep->in, T, prep->K,
+                                     const_cast<float*>(prep->xsum), st),
+                   "route + input kernel", err, len))
+      return NKT_ERR;
+    if (prep_done) *prep_done = true;
+  } else if (prep && h->act_bf16) {
     if (!check_hip(launch_route_prep_f16(logits, T, h->E, h->k, h->flags, ids, wts, prep->in, T, prep->K,
                                          const_cast<float*>(prep->xsum), prep->in16, prep->xinv, st),
                    "route + input kernel", err, len))
@@ -539,8 +546,8 @@ int do_router_logits(Handle* h, const void* x, int T, void* ws, const WsLayout& 
 // positions, the prefill form for its tiles, the tiled form otherwise.
 // The prefill form's gate_up first sums the activations per 128-wide group
 // (int formats; the down projection reads the sums gate_up writes).
-// prep_done: the int8 gate_up's fp16 input copy and group sums are already
-// made (by the routing launch).
+// prep_done: the gate_up's input preparation (int8: fp16 copy and group sums,
+// int4: group sums) is already made (by the routing launch).
 hipError_t launch_expert_gemm(const Handle* h, const GemmArgs& a, int phase, int bm, int tiles,
                               hipStream_t st, const KernelTimer* tm = nullptr, bool prep_done = false) {
   if (bm == 16 && gemv_supported(h->wf, phase, a.N, a.K, a.I)) return launch_gemv(a, h->wf, phase, tiles, st, tm);
@@ -553,7 +560,7 @@ hipError_t launch_expert_gemm(const Handle* h, const GemmArgs& a, int phase, int
         e = prep_done ? hipSuccess : launch_prep_f16(a.in, rows_in, a.K, const_cast<float*>(a.xsum), a.in16, a.xinv, st);
         b.in = a.in16;
       } else {
-        e = launch_group_sums(a.in, rows_in, a.K, const_cast<float*>(a.xsum), st);
+        e = prep_done ? hipSuccess : launch_group_sums(a.in, rows_in, a.K, const_cast<float*>(a.xsum), st);
         b.xinv = nullptr;
       }
       if (e != hipSuccess) return e;
@@ -880,16 +887,21 @@ int run_layer(Handle* h, const void* x, int T, void* out, void* ws, const WsLayo
     return NKT_OK;
   }
   // given logits and the int8 prefill gate_up on the fp16 matrix cores: its
-  // input copy is made in the routing launch
+  // input copy is made in the routing launch; the int4 gate_up's group sums
+  // likewise (Qwen3 int4 T = 203 / 2048
+  // 91.8 / 254.4 -> 87.8 / 245.6 us per layer)
   const GemmArgs g = expert_args(h, PHASE_GATE_UP, false, x, ws, L, T);
   const bool prep_in_route = logits && L.bm == kPrefillTileM && g.in16 && g.xinv &&
                              gemm2_supported(h->wf, PHASE_GATE_UP, g.N, g.K, g.I) && gemm2_i8_pipeline(g, h->wf);
+  const bool sums_in_route = logits && L.bm == kPrefillTileM && h->wf == WF_I4 &&
+                             gemm2_supported(h->wf, PHASE_GATE_UP, g.N, g.K, g.I);
   bool prep_done = false;
   // a few tokens from given logits: routing inside the gate_up launch
   const bool sr = sr_ok(h, T, L, logits, chunks);
   int rc = sr ? do_sr_gate_up(h, x, logits, T, ws, L, st, err, len)
               : prep_in_route ? do_route(h, logits, T, ws, L, st, err, len, &g, &prep_done,
                                          h->Is > 0 && chunks == 0 && allow_side && !side)
+              : sums_in_route ? do_route(h, logits, T, ws, L, st, err, len, &g, &prep_done)
                               : route();
   // a shared expert in the prefill form forks here, once the routing launch
   // has made the fp16 input copy both expert GEMMs read: its launches (a
@@ -899,7 +911,7 @@ int run_layer(Handle* h, const void* x, int T, void* out, void* ws, const WsLayo
   // the shared expert's prefill down in K parts (shared_down_parts), whether
   // it forks or stays on st
   const int parts = chunks == 0 && !side ? shared_down_parts(h, L, T) : 1;
-  const bool late_ok = (prep_done && L.bm_shared != kTileSrcCols && side_stream_ready(h, st)) ||
+  const bool late_ok = (prep_in_route && prep_done && L.bm_shared != kTileSrcCols && side_stream_ready(h, st)) ||
                        (x_from_route && shared_side_ready(h, T, L, st));
   if (rc == NKT_OK && allow_side && !side && h->Is > 0 && chunks == 0 && late_ok) {
     lk.lock();

@@ -817,9 +817,10 @@ __global__ void __launch_bounds__(256, 2) gemm2_bf16_kernel(GemmArgs a, int n_sl
 // Per-row sums of each 128-wide K group of a bf16 matrix [rows, K] -> fp32
 // [rows, K/128].  One wave per row; lane l adds its 8 consecutive values,
 // then the 16 lanes of a group reduce by xor butterfly (8, 4, 2, 1).
-__global__ void __launch_bounds__(256) group_sums_kernel(const uint16_t* __restrict__ x, int rows, int K,
-                                                         float* __restrict__ out) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+// block: this launch's index of the workgroup (four rows).
+__device__ __forceinline__ void group_sums_rows(const uint16_t* __restrict__ x, int rows, int K,
+                                                float* __restrict__ out, int block) {
+  const int row = block * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
   const uint16_t* xr = x + (int64_t)row * K;
@@ -841,6 +842,11 @@ __global__ void __launch_bounds__(256) group_sums_kernel(const uint16_t* __restr
     s += __shfl_xor(s, 1);
     if ((lane & 15) == 0 && g < G) out[(int64_t)row * G + g] = s;
   }
+}
+
+__global__ void __launch_bounds__(256) group_sums_kernel(const uint16_t* __restrict__ x, int rows, int K,
+                                                         float* __restrict__ out) {
+  group_sums_rows(x, rows, K, out, blockIdx.x);
 }
 
 // the int8 pipeline addresses its operands with 32-bit buffer offsets
@@ -1235,6 +1241,60 @@ __global__ void __launch_bounds__(256) route_prep_f16_kernel(const uint16_t* __r
     ids_out[(int64_t)t * k + lane] = id;
     w_out[(int64_t)t * k + lane] = w;
   }
+}
+
+// K1 and the int4 gate_up's group sums (as group_sums_kernel) in one launch,
+// split over the workgroups as route_prep_f16_kernel.  Bound by launch
+// latency: the two read 0.05 - 1 MB and 0.8 - 8 MB and each took 4 - 5 us of
+// its own (Qwen3 int4 T = 203 / 2048), with a gap between them.
+template <int VPL>
+__global__ void __launch_bounds__(256) route_sums_kernel(const uint16_t* __restrict__ logits, int T, int E, int k,
+                                                         unsigned flags, int32_t* __restrict__ ids_out,
+                                                         float* __restrict__ w_out, int route_blocks,
+                                                         const uint16_t* __restrict__ x, int rows, int K,
+                                                         float* __restrict__ sums) {
+  __shared__ float sv[4][kMaxTopK];
+  __shared__ int si[4][kMaxTopK];
+  if ((int)blockIdx.x >= route_blocks) {
+    group_sums_rows(x, rows, K, sums, blockIdx.x - route_blocks);
+    return;
+  }
+  const int wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + wave;
+  if (t >= T) return;
+  int id;
+  float w;
+  route_token<VPL, true>(logits, t, E, k, flags, sv[wave], si[wave], &id, &w);
+  if (lane < k) {
+    ids_out[(int64_t)t * k + lane] = id;
+    w_out[(int64_t)t * k + lane] = w;
+  }
+}
+
+hipError_t launch_route_sums(const void* logits, int T, int E, int k, unsigned flags, int32_t* ids, float* w,
+                             const void* x, int rows, int K, float* sums, hipStream_t stream) {
+  if (T <= 0 || rows <= 0) return hipErrorInvalidValue;
+  if (K % 128 != 0 || E <= 0 || E > 256) return hipErrorInvalidValue;
+  const int route_blocks = (T + 3) / 4;
+  const dim3 grid(route_blocks + (rows + 3) / 4), block(256);
+  const uint16_t* lg = (const uint16_t*)logits;
+  const uint16_t* xb = (const uint16_t*)x;
+#define NKT_RS_CASE(V)                                                                                            \
+  case V:                                                                                                         \
+    hipLaunchKernelGGL(route_sums_kernel<V>, grid, block, 0, stream, lg, T, E, k, flags, ids, w, route_blocks, xb, \
+                       rows, K, sums);                                                                            \
+    break;
+  switch ((E + 63) / 64) {
+    NKT_RS_CASE(1)
+    NKT_RS_CASE(2)
+    NKT_RS_CASE(3)
+    NKT_RS_CASE(4)
+    default:
+      return hipErrorInvalidValue;
+  }
+#undef NKT_RS_CASE
+  return hipGetLastError();
 }
 
 hipError_t launch_route_prep_f16(const void* logits, int T, int E, int k, unsigned flags, int32_t* ids, float* w,
