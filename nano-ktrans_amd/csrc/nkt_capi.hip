@@ -345,7 +345,6 @@ GemmArgs expert_args(const Handle* h, int phase, bool shared, const void* in, vo
     a.n_tiles = ws_ptr<int32_t>(ws, L, kWsNTiles);
     a.num_rows = T * h->k;
     if (phase == PHASE_GATE_UP && L.bm == kTileSrcCols) a.tile_src = ws_ptr<int32_t>(ws, L, kWsTileSrc);
-    a.narrow_tiles = (int64_t)T * h->k <= 48 * (int64_t)h->E;
   }
   const int64_t in_rows = (!shared && phase == PHASE_GATE_UP) ? T : a.num_rows;
   a.in_bytes = in_rows * K * (h->act_bf16 ? 2 : 4);
@@ -888,8 +887,8 @@ int run_layer(Handle* h, const void* x, int T, void* out, void* ws, const WsLayo
   }
   // given logits and the int8 prefill gate_up on the fp16 matrix cores: its
   // input copy is made in the routing launch; the int4 gate_up's group sums
-  // likewise (Qwen3 int4 T = 203 / 2048
-  // 91.8 / 254.4 -> 87.8 / 245.6 us per layer)
+  // likewise (Qwen3 int4 T = 203 / 2048 91.8 / 254.4
+  // -> 87.8 / 245.6 us per layer)
   const GemmArgs g = expert_args(h, PHASE_GATE_UP, false, x, ws, L, T);
   const bool prep_in_route = logits && L.bm == kPrefillTileM && g.in16 && g.xinv &&
                              gemm2_supported(h->wf, PHASE_GATE_UP, g.N, g.K, g.I) && gemm2_i8_pipeline(g, h->wf);

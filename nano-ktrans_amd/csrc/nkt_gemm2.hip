@@ -903,7 +903,7 @@ bool gemm2_supported(int wf, int phase, int N, int K, int I) {
 // allowed one), so one computes while the other waits.  Measured, eight
 // waves -> this: Mixtral T = 2048 gate_up 1081 -> 933 us (890 -> 1031
 // TFLOP/s), down 588 -> 536; Qwen3 T = 2048 gate_up 185 -> 164, down 124 ->
-// 96; Qwen3 T = 203 (narrow copies) gate_up 47.7 -> 44.4, down 33.4 -> 27.1.
+// 96; Qwen3 T = 203 (short-tile copies) gate_up 47.7 -> 44.4, down 33.4 -> 27.1.
 // KS = 2 (launch_gemm2's rule): eight waves, the second four on the second
 // half of K with buffers of their own, for launches too small to give every
 // CU two workgroups.
@@ -914,7 +914,7 @@ bool gemm2_supported(int wf, int phase, int N, int K, int I) {
 constexpr int kI4TokBytes = kBM * 256;
 constexpr int kI4SxBytes = 4 * 512;  // per wave: 256 B scales (128 used), 256 B group sums
 
-template <int PHASE, bool NARROW, int KS = 1>
+template <int PHASE, int KS>
 __global__ void __launch_bounds__(256 * KS, 2) gemm2_i4_kernel(GemmArgs a, int n_slabs, int sg) {
   constexpr int kWaves = 4;
   constexpr int kRT = 4;
@@ -1102,42 +1102,30 @@ __global__ void __launch_bounds__(256 * KS, 2) gemm2_i4_kernel(GemmArgs a, int n
     gemm2_epilogue<WF_I4, PHASE, kWaves>(a, acc, srcl, orow_l, hpart, xtot_l, xtot_l, wrow, sexp, it.row0, it.rows,
                                          it.slab, nullptr, PHASE == PHASE_DOWN ? tb2 + wave * 2304 : nullptr);
   };
-  // NARROW (experts average at most 48 positions): a tile of at most 16 / 32
-  // / 48 positions, an expert's last or only one, runs 1 / 2 / 3 of its 4
-  // column tiles (3: Qwen3 int4 T = 448 / 512 137.9 / 141.7 -> 129.1 / 133.3
-  // us, Mixtral T = 128 284.8 -> 265.7), an only tile with nt weight loads (T = 300 / 384 a further 124.5 /
-  // 130.9 -> 120.2 / 126.3 us with the nt copy; the 1-tile copy then T = 200
-  // / 256 / 300 114.9 / 116 / 117.5 -> 104.8 / 112.1 / 114.1 us).
-  // Measured: Qwen3 int4 T = 300 (even routing) 149 -> 124.6 us per layer;
-  // with the 1- and 2-tile copies the switch at 32 positions per expert
-  // measured best (Qwen3 int4 T = 448 / 512 153.6 / 147.6 -> 139 / 144 us,
-  // Mixtral T = 128 307 -> 292.5 against 24; at 48 T = 768 173.5 -> 178.5),
-  // with the 3-tile copies 48 (against 32: T = 640 / 768 154.5 / 172.6 ->
-  // 148 / 169.8, Mixtral T = 160 / 192 305.4 / 299.6 -> 279.5 / 289); where
-  // experts hold many full tiles the copies cost 1 - 5 % (Mixtral T = 2048,
-  // Qwen3 int4 Zipf T = 2048), hence the launch-wide switch
-  if constexpr (NARROW) {
-    // copy tag: column tiles | weight load policy << 4
-    const int urows = __builtin_amdgcn_readfirstlane(it.rows);
-    const bool only = __builtin_amdgcn_readfirstlane((int)it.only) != 0;
-    if (urows <= 16) {
-      if (only)
-        run(std::integral_constant<int, 1 | 2 << 4>{});
-      else
-        run(std::integral_constant<int, 1>{});
-    } else if (urows <= 32) {
-      if (only)
-        run(std::integral_constant<int, 2 | 2 << 4>{});
-      else
-        run(std::integral_constant<int, 2>{});
-    } else if (urows <= 48) {
-      if (only)
-        run(std::integral_constant<int, 3 | 2 << 4>{});
-      else
-        run(std::integral_constant<int, 3>{});
-    } else {
-      run(std::integral_constant<int, kCT>{});
-    }
+  // a tile of at most 16 / 32 / 48 positions, an expert's last or only one,
+  // runs 1 / 2 / 3 of its 4 column tiles, an only tile with nt weight loads
+  // (copy tag: column tiles | weight load policy << 4).  Measured against
+  // always 4 column tiles, us per layer: Qwen3 int4 T = 1000 / 2048 / 4096
+  // 164.2 / 247.5 / 411 -> 153.7 / 242 / 403.6, Zipf routing T = 4096 409.9 ->
+  // 400.9, Mixtral-8x7B T = 220 / 600 / 2048 293.8 / 557.9 / 1449 -> 274.1 /
+  // 529.4 / 1426, Qwen3 T = 700 (mostly short tiles either way) level.
+  const int urows = __builtin_amdgcn_readfirstlane(it.rows);
+  const bool only = __builtin_amdgcn_readfirstlane((int)it.only) != 0;
+  if (urows <= 16) {
+    if (only)
+      run(std::integral_constant<int, 1 | 2 << 4>{});
+    else
+      run(std::integral_constant<int, 1>{});
+  } else if (urows <= 32) {
+    if (only)
+      run(std::integral_constant<int, 2 | 2 << 4>{});
+    else
+      run(std::integral_constant<int, 2>{});
+  } else if (urows <= 48) {
+    if (only)
+      run(std::integral_constant<int, 3 | 2 << 4>{});
+    else
+      run(std::integral_constant<int, 3>{});
   } else {
     run(std::integral_constant<int, kCT>{});
   }
@@ -1369,7 +1357,7 @@ constexpr int gemm2_waves(int wf) { return wf == WF_I8 ? 4 : 8; }
 // stages on 16 slabs x 8 experts = 128 items) is the whole launch.  Measured,
 // Mixtral-8x7B int4, one part -> two, us per layer: T = 100 209 -> 190; eight
 // waves of 32 rows on all of K (before): T = 40 / 100 / 180 178 / 204 / 262
-// -> 167 / 190 / 241, T = 240 (the rule's edge) 324 -> 322.
+// -> 167 / 190 / 241, T = 220 300 -> 274.
 constexpr int64_t kI4SplitMaxItems = 256;
 
 hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hipStream_t stream,
@@ -1409,16 +1397,12 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
   }
   if (gemm2_i4_pipeline(a, wf)) {
     block = dim3(256);
-    if (phase == PHASE_GATE_UP && a.narrow_tiles)
-      launch_timed(gemm2_i4_kernel<PHASE_GATE_UP, true>, grid, block, 0, stream, tm, a, n_slabs, sg);
-    else if (phase == PHASE_GATE_UP)
-      launch_timed(gemm2_i4_kernel<PHASE_GATE_UP, false>, grid, block, 0, stream, tm, a, n_slabs, sg);
-    else if (a.narrow_tiles && items <= kI4SplitMaxItems && a.K % 256 == 0)
-      launch_timed(gemm2_i4_kernel<PHASE_DOWN, true, 2>, grid, dim3(512), 0, stream, tm, a, n_slabs, sg);
-    else if (a.narrow_tiles)
-      launch_timed(gemm2_i4_kernel<PHASE_DOWN, true>, grid, block, 0, stream, tm, a, n_slabs, sg);
+    if (phase == PHASE_GATE_UP)
+      launch_timed(gemm2_i4_kernel<PHASE_GATE_UP, 1>, grid, block, 0, stream, tm, a, n_slabs, sg);
+    else if (items <= kI4SplitMaxItems && a.K % 256 == 0)
+      launch_timed(gemm2_i4_kernel<PHASE_DOWN, 2>, grid, dim3(512), 0, stream, tm, a, n_slabs, sg);
     else
-      launch_timed(gemm2_i4_kernel<PHASE_DOWN, false>, grid, block, 0, stream, tm, a, n_slabs, sg);
+      launch_timed(gemm2_i4_kernel<PHASE_DOWN, 1>, grid, block, 0, stream, tm, a, n_slabs, sg);
     return hipGetLastError();
   }
   switch (wf) {

@@ -63,11 +63,6 @@ struct GemmArgs {
   // (tile, slab) item once per part; part p's fp32 partial rows go to
   // out + p num_rows N, and the combine adds the parts in order
   int k_parts;
-  // prefill int4, nonzero: a tile of at most 16 / 32 / 48 positions (an
-  // expert's last or only one) runs a copy of the pipeline over the first
-  // one / two / three of its four 16-position column tiles (set where experts
-  // average at most 48 positions)
-  int narrow_tiles;
   // single-token decode gate_up that routes its token itself
   // (route_logits != nullptr, [1, route_E] bf16): every workgroup runs K1
   // on the one row of logits, workgroup (0, 0) also writes K1's and K2's
