@@ -342,8 +342,8 @@ def kernel_form(w, T):
     int8 = 3.5 if w.shared else 4.5
     if avg <= {"int8_per_channel": int8, "int4_g128": 6 if w.I >= 8192 else 8}.get(w.wfmt, 12):
         return "gemv_kernel"
-    # int8 and int4 (bf16 activations, buffers under 4 GiB: every bench shape) have pipelined kernels
-    return {"int8_per_channel": "gemm2_i8_kernel", "int4_g128": "gemm2_i4_kernel"}.get(w.wfmt, "gemm2_kernel")
+    # bf16 activations, buffers under 2 GiB (every bench shape): the pipelined kernels
+    return {"int8_per_channel": "gemm2_i8_kernel", "int4_g128": "gemm2_i4_kernel"}.get(w.wfmt, "gemm2_bf16_kernel")
 
 
 def bench_workload(w, T, layers, router, steps, warmup, device):
@@ -634,13 +634,14 @@ def _phase_of(name):
     """gate_up / down from an expert-GEMM kernel's template arguments (None otherwise)."""
     import re
 
-    m = re.search(r"nkt::(gemv_kernel|gemm2_kernel|gemm_kernel|gemm2_i8_kernel|gemm2_i4_kernel)<([^>]*)>", name)
+    m = re.search(r"nkt::(gemv_kernel|gemm2_kernel|gemm_kernel|gemm2_i8_kernel|gemm2_i4_kernel|gemm2_bf16_kernel)<([^>]*)>", name)
     if not m:
         return None
     args = [a.strip() for a in m.group(2).split(",")]
     # template arguments: gemv_kernel<WF, PHASE, ...>, gemm2_kernel<WF, PHASE, NW>,
-    # gemm_kernel<WF, BM, NW, RT, PHASE, ...>, gemm2_i8_kernel<PHASE, F16>, gemm2_i4_kernel<PHASE, NARROW>
-    idx = {"gemm2_i8_kernel": 0, "gemm2_i4_kernel": 0, "gemm_kernel": 4}.get(m.group(1), 1)
+    # gemm_kernel<WF, BM, NW, RT, PHASE, ...>, gemm2_i8_kernel<PHASE, F16>, gemm2_i4_kernel<PHASE, KS>,
+    # gemm2_bf16_kernel<PHASE>
+    idx = {"gemm2_i8_kernel": 0, "gemm2_i4_kernel": 0, "gemm2_bf16_kernel": 0, "gemm_kernel": 4}.get(m.group(1), 1)
     val = args[idx].split(")")[-1]
     return "gate_up" if val == "0" else "down"
 
