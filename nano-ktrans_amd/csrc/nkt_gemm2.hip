@@ -10,9 +10,9 @@
 //   * gemm2_i8_kernel (int8): 4 waves, three-stage pipeline of 64-wide K
 //     stages (tokens direct-to-LDS, weights in a register ring), gate_up on
 //     the fp16 matrix cores;
-//   * gemm2_i4_kernel (int4 g128): 4 waves, three-stage pipeline of 128-wide
-//     K stages (tokens, scales and group sums direct-to-LDS, weights in a
-//     ring of two register stages);
+//   * gemm2_i4_kernel (int4 g128): 4 or 8 waves, three-stage pipeline of
+//     128-wide K stages (tokens, scales and group sums direct-to-LDS, weights
+//     in a ring of two register stages);
 //   * gemm2_bf16_kernel (bf16): the int8 pipeline's form, two weight blocks
 //     per row tile and stage;
 //   * gemm2_kernel (operands past the pipelines' 32-bit buffer offsets): the
@@ -247,6 +247,10 @@ __device__ __forceinline__ void gemm2_epilogue(const GemmArgs& a, f32x4 (&acc)[1
   if (PHASE == PHASE_GATE_UP) {
     const int hcol0 = slab * 128 + wave * (128 / kWaves);
     constexpr int HR = kRT / 2;
+    // h's group sums (hsum): int4 per 16-column tile, whichever wave holds it
+    // (its four- and eight-wave forms give the same bits), through LDS
+    // (stage: [tile][position][4 lanes], no shuffles); the others per wave
+    float* const hp = (float*)stage;
     f32x4 sg[HR], su[HR];
     if (WF == WF_I8) {
 #pragma unroll
@@ -261,6 +265,7 @@ __device__ __forceinline__ void gemm2_epilogue(const GemmArgs& a, f32x4 (&acc)[1
       float part = 0.f;
 #pragma unroll
       for (int r = 0; r < HR; ++r) {
+        if (WF == WF_I4) part = 0.f;
         f32x4 gv = acc[r][c], uv = acc[r + HR][c];
         if (WF == WF_I8) {
           gv *= sg[r];
@@ -276,18 +281,31 @@ __device__ __forceinline__ void gemm2_epilogue(const GemmArgs& a, f32x4 (&acc)[1
         part += hb[3];
         // h goes out directly: staged like y below it measured ~2 % slower
         if (pl < rows) *(u32x2*)((uint16_t*)a.out + (int64_t)(row0 + pl) * a.I + hcol0 + r * 16 + rq) = pk;
+        if (WF == WF_I4) hp[((wave * HR + r) * kBM + pl) * 4 + (lane >> 4)] = part;
       }
-      // the 4 lanes holding one position's columns: fixed-order butterfly
-      part += __shfl_xor(part, 16);
-      part += __shfl_xor(part, 32);
-      if (lane < 16) hpart[wave][pl] = part;
+      if (WF != WF_I4) {
+        // the 4 lanes holding one position's columns: fixed-order butterfly
+        part += __shfl_xor(part, 16);
+        part += __shfl_xor(part, 32);
+        if (lane < 16) hpart[wave][pl] = part;
+      }
     }
     if (a.hsum) {
       lds_barrier();
       if (tid < kBM && tid < rows) {
-        float s = hpart[0][tid];
+        float s;
+        if (WF == WF_I4) {
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) s += hpart[w][tid];
+          for (int t = 0; t < 8; ++t) {
+            const f32x4 q = *(const f32x4*)(hp + (t * kBM + tid) * 4);
+            const float v = (q[0] + q[1]) + (q[2] + q[3]);
+            s = t == 0 ? v : s + v;
+          }
+        } else {
+          s = hpart[0][tid];
+#pragma unroll
+          for (int w = 1; w < kWaves; ++w) s += hpart[w][tid];
+        }
         a.hsum[(int64_t)(row0 + tid) * (a.I / 128) + slab] = s;
       }
     }
@@ -537,7 +555,8 @@ __global__ void __launch_bounds__(64 * kWaves, 2) gemm2_kernel(GemmArgs a, int n
   }
   __syncthreads();
 
-  gemm2_epilogue<WF, PHASE, kWaves>(a, acc, srcl, orow_l, hpart, xtot_l, xtot_l, wrow, sexp, row0, rows, slab);
+  gemm2_epilogue<WF, PHASE, kWaves>(a, acc, srcl, orow_l, hpart, xtot_l, xtot_l, wrow, sexp, row0, rows, slab,
+                                    nullptr, WF == WF_I4 && PHASE == PHASE_GATE_UP ? bt0 : nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -875,80 +894,77 @@ bool gemm2_supported(int wf, int phase, int N, int K, int I) {
 }
 
 // ---------------------------------------------------------------------------
-// int4 g128 weights, three-stage pipeline.  Same tile, work order and scaling
-// sequence as gemm2_kernel<WF_I4, ...>; 4 waves of four 16-row tiles each,
-// two workgroups per CU; K advances one 128-wide scale group per stage:
+// int4 g128 weights, three-stage pipeline on the int8 pipeline's tile and
+// work order, as four waves of four 16-row tiles (two workgroups per CU) or
+// eight waves of two; K advances one 128-wide scale group per stage:
 //   * tokens: 64 positions x 256 B per stage reach one of three LDS buffers
-//     by direct-to-LDS buffer loads (16 loads of 4 positions, 4 per wave);
+//     by direct-to-LDS buffer loads (16 loads of 4 positions over the waves);
 //     lane l carries position 4 i + l / 16 into slot l % 16 of that
 //     position's row, fetched from chunk (l % 16) ^ (position % 16), so the
 //     MFMA operand reads of 16 consecutive positions cover all 64 banks;
-//   * each wave's four 1 KiB weight blocks go by buffer loads straight into
-//     one of two register stages; their bf16 scales (lanes 0-31, 4 bytes
-//     each) and the 64 positions' activation group sums (4 bytes per lane)
-//     reach the wave's own slice of a small LDS buffer by direct-to-LDS
-//     loads;
-//   * step x: wait for this wave's loads of stage x (all but the newest 10,
-//     the loads of stage x + 1), one LDS-only barrier (every wave is also
-//     done reading stage x - 1's buffers), start stage x + 2's token loads
-//     into those buffers, dequantise stage x's weights, start stage x + 2's
-//     weight loads into the registers that frees, then column tile by column
-//     tile: four MFMAs per row tile into a temporary that starts at the code
-//     offset, the 4 temporaries advancing together, then scaled into the
-//     accumulators.
+//   * each wave's 1 KiB weight blocks (one per row tile) go by buffer loads
+//     straight into one of two register stages; their bf16 scales (8 lanes
+//     per row tile, 4 bytes each) and the 64 positions' activation group sums
+//     (4 bytes per lane) reach the wave's own slice of a small LDS buffer by
+//     direct-to-LDS loads;
+//   * step x: wait for this wave's loads of stage x (all but the newest
+//     kStepLoads, those of stage x + 1), one LDS-only barrier (every wave is
+//     also done reading stage x - 1's buffers), start stage x + 2's token
+//     loads into those buffers, dequantise stage x's weights, start stage
+//     x + 2's weight loads into the registers that frees, then four MFMAs per
+//     (row tile, column tile) into a temporary that starts at the code
+//     offset, scaled into the accumulators.
+// Both forms, whatever the launch, sum an output's K groups in ascending
+// order and h's group sums over 16-column tiles in ascending order, so an
+// int4 prefill row has the same bits in every batch.
 // What bounds it: neither HBM nor one unit, but the waits a stage's barrier
 // and an item's start and end leave.  Four waves of 64 rows read each token
-// fragment from LDS half as often as eight waves of 32, and fit two
-// workgroups per CU (251 VGPRs at 2 waves per SIMD; eight waves of 210
-// allowed one), so one computes while the other waits.  Measured, eight
-// waves -> this: Mixtral T = 2048 gate_up 1081 -> 933 us (890 -> 1031
-// TFLOP/s), down 588 -> 536; Qwen3 T = 2048 gate_up 185 -> 164, down 124 ->
-// 96; Qwen3 T = 203 (short-tile copies) gate_up 47.7 -> 44.4, down 33.4 -> 27.1.
-// KS = 2 (launch_gemm2's rule): eight waves, the second four on the second
-// half of K with buffers of their own, for launches too small to give every
-// CU two workgroups.
+// fragment from LDS half as often as eight waves of 32 and fit two
+// workgroups per CU (251 VGPRs at 2 waves per SIMD), so one computes while
+// the other waits: at Mixtral T = 2000 gate_up 853 us (four) against 999
+// (eight), down 466 / 477, Qwen3 T = 2048 gate_up 130 / 153, down 81 / 99.
+// Where a launch has no second workgroup for a CU, eight waves on the one
+// workgroup finish it sooner (launch_gemm2's rule and figures).
 // Loads past the last stage take an out-of-range buffer offset (no
-// traffic), so every step issues the same 10.  Six LDS objects: the compiler
-// tells a direct-to-LDS load into one from reads of another.
+// traffic), so every step issues the same loads.  Six LDS objects: the
+// compiler tells a direct-to-LDS load into one from reads of another.
 // ---------------------------------------------------------------------------
 constexpr int kI4TokBytes = kBM * 256;
-constexpr int kI4SxBytes = 4 * 512;  // per wave: 256 B scales (128 used), 256 B group sums
+constexpr int kI4SxBytes = 512;  // per wave: 256 B scales (4 waves: 128 used, 8 waves: 64), 256 B group sums
 
-template <int PHASE, int KS>
-__global__ void __launch_bounds__(256 * KS, 2) gemm2_i4_kernel(GemmArgs a, int n_slabs, int sg) {
-  constexpr int kWaves = 4;
-  constexpr int kRT = 4;
-  constexpr int kStepLoads = 10;  // a stage's loads per wave: 4 token, 4 weight, scales, group sums
-  __shared__ __attribute__((aligned(1024))) uint8_t tb0[KS * kI4TokBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t tb1[KS * kI4TokBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t tb2[KS * kI4TokBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t sx0[KS * kI4SxBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t sx1[KS * kI4SxBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t sx2[KS * kI4SxBytes];
+template <int PHASE, int kWaves>
+__device__ __forceinline__ void gemm2_stage128(const GemmArgs& a, int n_slabs, int sg) {
+  static_assert(kWaves == 4 || kWaves == 8, "four or two row tiles per wave");
+  constexpr int kRT = 16 / kWaves;            // 16-row weight tiles per wave
+  constexpr int kTL = 16 / kWaves;            // token loads (4 positions each) per wave and stage
+  constexpr int kStepLoads = kTL + kRT + 2;   // a stage's loads per wave: tokens, weights, scales, group sums
+  __shared__ __attribute__((aligned(1024))) uint8_t tb0[kI4TokBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t tb1[kI4TokBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t tb2[kI4TokBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t sx0[kWaves * kI4SxBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t sx1[kWaves * kI4SxBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t sx2[kWaves * kI4SxBytes];
   __shared__ int srcl[kBM];
   __shared__ int orow_l[kBM];
-  __shared__ float hpart[kWaves][kBM];
+  __shared__ float hpart[kWaves][kBM];  // down
   __shared__ float xtot_l[kBM];
 
   TileItem it;
   if (!gemm2_item(a, n_slabs, sg, it)) return;
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % kWaves;
-  const int part = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;  // this wave's K part
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   gemm2_sources(a, it, srcl, orow_l);
   __syncthreads();
 
   const uint16_t* sexp = a.scales + (int64_t)it.expert * a.s_expert_elems;
-  const int Grow = a.K / 128;  // scale groups = 1 KiB blocks per 16-row block
-  const int G = Grow / KS;     // stages of this wave's K part
-  const int g0 = part * G;
+  const int G = a.K / 128;  // stages = scale groups = 1 KiB blocks per 16-row block
   const int rows_in = (int)(a.in_bytes / ((int64_t)a.K * 2));
   const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(a.w + (int64_t)it.expert * a.w_expert_bytes), (short)0, (int)a.w_expert_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t sres =
       __builtin_amdgcn_make_buffer_rsrc((void*)sexp, (short)0, (int)(a.s_expert_elems * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t xres =
-      __builtin_amdgcn_make_buffer_rsrc((void*)a.xsum, (short)0, rows_in * Grow * 4, 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.xsum, (short)0, rows_in * G * 4, 0x00020000);
   const __amdgpu_buffer_rsrc_t tres = __builtin_amdgcn_make_buffer_rsrc((void*)a.in, (short)0, (int)a.in_bytes, 0x00020000);
   int wrow[kRT];
   uint32_t wsrc[kRT];
@@ -958,23 +974,24 @@ __global__ void __launch_bounds__(256 * KS, 2) gemm2_i4_kernel(GemmArgs a, int n
       wrow[r] = (r < kRT / 2 ? 0 : a.I) + it.slab * 128 + wave * (128 / kWaves) + (r % (kRT / 2)) * 16;
     else
       wrow[r] = it.slab * 256 + wave * (256 / kWaves) + r * 16;
-    wsrc[r] = ((uint32_t)(wrow[r] >> 4) * (uint32_t)Grow + (uint32_t)g0) * 1024u;  // the same in every lane
+    wsrc[r] = (uint32_t)(wrow[r] >> 4) * (uint32_t)G * 1024u;  // the same in every lane
   }
-  // scale lane (lanes 32-63 repeat lanes 0-31): row tile (l % 32) / 8, 4-byte piece l % 8
-  const int sl = (lane >> 3) & 3;
-  const int srow = sl == 0 ? wrow[0] : sl == 1 ? wrow[1] : sl == 2 ? wrow[2] : wrow[3];
-  const uint32_t ssrc = ((uint32_t)(srow >> 4) * (uint32_t)Grow + (uint32_t)g0) * 32u + (lane & 7) * 4u;
-  const uint32_t xsrc = ((uint32_t)srcl[lane] * (uint32_t)Grow + (uint32_t)g0) * 4u;
-  uint32_t tsrc[4];
+  // scale lane (lanes past 8 kRT repeat the first): row tile (l / 8) % kRT, 4-byte piece l % 8
+  const int sl = (lane >> 3) & (kRT - 1);
+  int srow = wrow[0];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int p = 16 * wave + 4 * j + (lane >> 4);
+  for (int r = 1; r < kRT; ++r) srow = sl == r ? wrow[r] : srow;
+  const uint32_t ssrc = (uint32_t)(srow >> 4) * (uint32_t)G * 32u + (lane & 7) * 4u;
+  const uint32_t xsrc = (uint32_t)srcl[lane] * (uint32_t)G * 4u;
+  uint32_t tsrc[kTL];
+#pragma unroll
+  for (int j = 0; j < kTL; ++j) {
+    const int p = 4 * kTL * wave + 4 * j + (lane >> 4);
     const int chunk = (lane & 15) ^ (p & 15);
-    tsrc[j] = (uint32_t)srcl[p] * (uint32_t)a.K * 2u + (uint32_t)g0 * 256u + chunk * 16u;
+    tsrc[j] = (uint32_t)srcl[p] * (uint32_t)a.K * 2u + chunk * 16u;
   }
-  const int tpart = part * kI4TokBytes;                // this K part's token buffer
-  const int tofs = tpart + wave * 4096;                // this wave's slice of it
-  const int sofs = part * kI4SxBytes + wave * 512;     // and of a scale / group-sum buffer
+  const int tofs = wave * kTL * 1024;    // this wave's slice of a token buffer
+  const int sofs = wave * kI4SxBytes;    // and of a scale / group-sum buffer
 
   // stage st's token, scale and group-sum loads, and its weight loads with
   // the copy's load policy (tag >> 4: nt for an expert's only tile); st >= G:
@@ -982,7 +999,7 @@ __global__ void __launch_bounds__(256 * KS, 2) gemm2_i4_kernel(GemmArgs a, int n
   auto issue_tok = [&](int st, uint8_t* tb, uint8_t* sx) __attribute__((always_inline)) {
     const bool live = st < G;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < kTL; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(tres, (__attribute__((address_space(3))) void*)(tb + tofs + j * 1024),
                                                16, live ? tsrc[j] : kI8Skip, live ? st * 256 : 0, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(sres, (__attribute__((address_space(3))) void*)(sx + sofs), 4,
@@ -1005,35 +1022,62 @@ __global__ void __launch_bounds__(256 * KS, 2) gemm2_i4_kernel(GemmArgs a, int n
 #pragma unroll
     for (int c = 0; c < kCT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // one column tile at a time: its 4 row tiles' temporaries advance one K
-  // step at a time (4 independent chains; the CU's second workgroup fills
-  // what they leave), then the group scales; only the first NC column tiles
+  // Only the first NC column tiles.  Four waves: one column tile at a time,
+  // its 4 row tiles' temporaries advance one K step at a time (4 independent
+  // chains; the CU's second workgroup fills what they leave), then the group
+  // scales.  Eight waves: all (row tile, column tile) temporaries together.
+  // Either way each element takes the same operations in the same order.
   auto compute = [&](auto nc, const u32x4 (&ad)[kRT][4], const uint8_t* tb, const uint8_t* sx) __attribute__((always_inline)) {
     constexpr int NC = decltype(nc)::value & 15;
     f32x4 sc[kRT];
 #pragma unroll
     for (int r = 0; r < kRT; ++r) sc[r] = bf16x4_to_f32(*(const u32x2*)(sx + sofs + r * 32 + (lane >> 4) * 8));
-    u32x4 bf[2][4];
     auto read_b = [&](u32x4 (&f)[4], int c) __attribute__((always_inline)) {
       const int p = c * 16 + (lane & 15);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) f[s] = *(const u32x4*)(tb + tpart + p * 256 + (((4 * s + (lane >> 4)) ^ (p & 15)) * 16));
+      for (int s = 0; s < 4; ++s) f[s] = *(const u32x4*)(tb + p * 256 + (((4 * s + (lane >> 4)) ^ (p & 15)) * 16));
     };
-    read_b(bf[0], 0);
+    auto offset = [&](int c) __attribute__((always_inline)) {
+      return -136.0f * *(const float*)(sx + sofs + 256 + (c * 16 + (lane & 15)) * 4);
+    };
+    if constexpr (kWaves == 4) {
+      u32x4 bf[2][4];
+      read_b(bf[0], 0);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      if (c + 1 < NC) read_b(bf[(c + 1) & 1], c + 1);
-      const float cv = -136.0f * *(const float*)(sx + sofs + 256 + (c * 16 + (lane & 15)) * 4);
-      f32x4 tmp[kRT];
+      for (int c = 0; c < NC; ++c) {
+        if (c + 1 < NC) read_b(bf[(c + 1) & 1], c + 1);
+        const float cv = offset(c);
+        f32x4 tmp[kRT];
 #pragma unroll
-      for (int r = 0; r < kRT; ++r) tmp[r] = f32x4{cv, cv, cv, cv};
+        for (int r = 0; r < kRT; ++r) tmp[r] = f32x4{cv, cv, cv, cv};
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int r = 0; r < kRT; ++r) tmp[r] = mfma_bf16(ad[r][s], bf[c & 1][s], tmp[r]);
+#pragma unroll
+        for (int r = 0; r < kRT; ++r) acc[r][c] += sc[r] * tmp[r];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      u32x4 bf[NC][4];
+      f32x4 tmp[kRT][NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        read_b(bf[c], c);
+        const float cv = offset(c);
+#pragma unroll
+        for (int r = 0; r < kRT; ++r) tmp[r][c] = f32x4{cv, cv, cv, cv};
+      }
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int r = 0; r < kRT; ++r) tmp[r] = mfma_bf16(ad[r][s], bf[c & 1][s], tmp[r]);
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int r = 0; r < kRT; ++r) acc[r][c] += sc[r] * tmp[r];
-      __builtin_amdgcn_sched_barrier(0);
+          for (int r = 0; r < kRT; ++r) tmp[r][c] = mfma_bf16(ad[r][s], bf[c][s], tmp[r][c]);
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int r = 0; r < kRT; ++r) acc[r][c] += sc[r] * tmp[r][c];
     }
   };
 
@@ -1079,28 +1123,10 @@ __global__ void __launch_bounds__(256 * KS, 2) gemm2_i4_kernel(GemmArgs a, int n
     if (rest >= 5) step(nc, w0, tb1, sx1, tb0, sx0, x + 4);
     wait_vmem();  // out-of-range loads past the last stage land before the LDS is reused
     __syncthreads();
-    if constexpr (KS > 1) {
-      // the second K part's sums reach the first through the token buffers
-      // (16 bytes per lane, one 1 KiB row per wave and tile); its waves end
-      auto slot = [&](int r, int c) __attribute__((always_inline)) {
-        return (f32x4*)((r < 2 ? tb0 : tb1) + (((r & 1) * kCT + c) * kWaves + wave) * 1024 + lane * 16);
-      };
-      if (part == 1) {
-#pragma unroll
-        for (int r = 0; r < kRT; ++r)
-#pragma unroll
-          for (int c = 0; c < kCT; ++c) *slot(r, c) = acc[r][c];
-      }
-      __syncthreads();
-      if (part == 1) return;
-#pragma unroll
-      for (int r = 0; r < kRT; ++r)
-#pragma unroll
-        for (int c = 0; c < kCT; ++c) acc[r][c] += *slot(r, c);
-    }
-    // down's compact y staging: 16 rows of 144 B per wave in a token buffer
+    // in a token buffer: down's compact y staging, 16 rows of 32 kRT + 16
+    // bytes per wave; gate_up's 8 KiB of h's partial group sums
     gemm2_epilogue<WF_I4, PHASE, kWaves>(a, acc, srcl, orow_l, hpart, xtot_l, xtot_l, wrow, sexp, it.row0, it.rows,
-                                         it.slab, nullptr, PHASE == PHASE_DOWN ? tb2 + wave * 2304 : nullptr);
+                                         it.slab, nullptr, PHASE == PHASE_DOWN ? tb2 + wave * 16 * (32 * kRT + 16) : tb2);
   };
   // a tile of at most 16 / 32 / 48 positions, an expert's last or only one,
   // runs 1 / 2 / 3 of its 4 column tiles, an only tile with nt weight loads
@@ -1129,6 +1155,11 @@ __global__ void __launch_bounds__(256 * KS, 2) gemm2_i4_kernel(GemmArgs a, int n
   } else {
     run(std::integral_constant<int, kCT>{});
   }
+}
+
+template <int PHASE, int kWaves>
+__global__ void __launch_bounds__(64 * kWaves, 2) gemm2_i4_kernel(GemmArgs a, int n_slabs, int sg) {
+  gemm2_stage128<PHASE, kWaves>(a, n_slabs, sg);
 }
 
 // Input of the int8 gate_up on the fp16 matrix cores, one wave per row: the
@@ -1350,15 +1381,33 @@ hipError_t launch_group_sums(const void* x, int rows, int K, float* out, hipStre
 // int4 adds per-group scale temporaries) and removes their spills.
 constexpr int gemm2_waves(int wf) { return wf == WF_I8 ? 4 : 8; }
 
-// The int4 down runs its K in two halves on eight waves (KS = 2) while the
-// launch has at most this many (token tile, weight slab) items (counted with
-// the tile list's upper bound): one workgroup per CU or fewer, so two
-// four-wave workgroups never share a CU and the long K loop (Mixtral: 112
-// stages on 16 slabs x 8 experts = 128 items) is the whole launch.  Measured,
-// Mixtral-8x7B int4, one part -> two, us per layer: T = 100 209 -> 190; eight
-// waves of 32 rows on all of K (before): T = 40 / 100 / 180 178 / 204 / 262
-// -> 167 / 190 / 241, T = 220 300 -> 274.
-constexpr int64_t kI4SplitMaxItems = 256;
+// Tiles the launch can expect: exact for a dense launch; for a tile list
+// (max_tiles is its upper bound, all full tiles and one more per expert) from
+// the mean positions per expert -- one tile each up to 50 (at 64 half of the
+// experts hold two), from 64 on the full ones and half a tile more.
+static double gemm2_expected_tiles(const GemmArgs& a, int max_tiles) {
+  if (!a.n_tiles) return max_tiles;
+  const int full = a.num_rows / kBM;
+  const double experts = max_tiles - full, n = a.num_rows / experts;
+  if (n <= 50.0) return experts;
+  return n < kBM ? experts * (1.0 + (n - 50.0) / (2.0 * (kBM - 50.0))) : a.num_rows / (double)kBM + 0.5 * experts;
+}
+
+// Eight waves per workgroup instead of four (the results are the same bit for
+// bit).  int4: while the launch has at most one (tile, slab) item per CU -- a
+// lone four-wave workgroup leaves its SIMDs one wave each.  Measured, us, four
+// waves against eight, weights from HBM: gate_up H = 2048 I = 768, 16 experts,
+// 96 / 144 / 240 items 24.4 / 28.6 / 29.4 against 20.2 / 23.7 / 24.4; H = I =
+// 4096, 8 experts, 256 items 43.5 / 36.7; Mixtral-8x7B down 128 / 192 / 244
+// items 121 / 152 / 154 against 97 / 121 / 119.  Past one item per CU two
+// four-wave workgroups share it: gate_up 319 / 366 / 480 items 37.0 / 37.8 /
+// 39.1 against 42.0 / 42.8 / 43.3, down 320 items (H = 4096 I = 4096) 63.0 /
+// 72.6.
+constexpr double kGemm2Cus = 256.0;
+
+static bool gemm2_eight_waves(const GemmArgs& a, int wf, int n_slabs, int max_tiles) {
+  return wf == WF_I4 && n_slabs * gemm2_expected_tiles(a, max_tiles) <= kGemm2Cus;
+}
 
 hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hipStream_t stream,
                         const KernelTimer* tm) {
@@ -1396,13 +1445,16 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
     return hipGetLastError();
   }
   if (gemm2_i4_pipeline(a, wf)) {
-    block = dim3(256);
-    if (phase == PHASE_GATE_UP)
-      launch_timed(gemm2_i4_kernel<PHASE_GATE_UP, 1>, grid, block, 0, stream, tm, a, n_slabs, sg);
-    else if (items <= kI4SplitMaxItems && a.K % 256 == 0)
-      launch_timed(gemm2_i4_kernel<PHASE_DOWN, 2>, grid, dim3(512), 0, stream, tm, a, n_slabs, sg);
+    const bool w8 = gemm2_eight_waves(a, wf, n_slabs, max_tiles);
+    block = dim3(w8 ? 512 : 256);
+    if (phase == PHASE_GATE_UP && w8)
+      launch_timed(gemm2_i4_kernel<PHASE_GATE_UP, 8>, grid, block, 0, stream, tm, a, n_slabs, sg);
+    else if (phase == PHASE_GATE_UP)
+      launch_timed(gemm2_i4_kernel<PHASE_GATE_UP, 4>, grid, block, 0, stream, tm, a, n_slabs, sg);
+    else if (w8)
+      launch_timed(gemm2_i4_kernel<PHASE_DOWN, 8>, grid, block, 0, stream, tm, a, n_slabs, sg);
     else
-      launch_timed(gemm2_i4_kernel<PHASE_DOWN, 1>, grid, block, 0, stream, tm, a, n_slabs, sg);
+      launch_timed(gemm2_i4_kernel<PHASE_DOWN, 4>, grid, block, 0, stream, tm, a, n_slabs, sg);
     return hipGetLastError();
   }
   switch (wf) {

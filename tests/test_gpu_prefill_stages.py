@@ -29,3 +29,22 @@ def test_stage_and_tile_remainders(gpu_device, wfmt, H, I):
         torch.cuda.synchronize()
         ref = oracle_forward(layer, x, logits)
         compare(out.float().cpu().numpy(), ref, cfg)
+
+
+def test_int4_rows_same_bits_in_every_batch(gpu_device):
+    """An int4 prefill row does not depend on the batch it is in: few experts
+    at token counts on both sides of one (tile, slab) item per CU, where
+    gate_up (16 slabs) and then down (8 slabs) go from eight waves per
+    workgroup to four -- both on eight up to T = 256 (at most 192 items),
+    gate_up on four at 400, both at 1024 -- give bit-identical prefixes."""
+    cfg = replace(CONFIGS["qwen3_int4"], name="few_experts_int4", H=2048, I=2048, E=8, k=2)
+    layer = build_layer(cfg, device="cuda")
+    native = native_layer(layer, torch.device("cuda"))
+    x, logits = build_inputs(layer, 1024, seed=3, device="cuda")
+    full = native.forward(x, logits).clone()
+    compare(full[:97].float().cpu().numpy(), oracle_forward(layer, x[:97], logits[:97]), cfg)
+    for T in (33, 64, 180, 256, 400, 900):
+        assert not cfg.decode_form(T)
+        part = native.forward(x[:T].contiguous(), logits[:T].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(full[:T], part), f"T = {T}"
