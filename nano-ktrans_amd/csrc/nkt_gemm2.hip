@@ -15,8 +15,9 @@
 //     in a ring of two register stages);
 //   * gemm2_bf16_kernel (bf16): the int8 pipeline's form, two weight blocks
 //     per row tile and stage;
-//   * gemm2_kernel (operands past the pipelines' 32-bit buffer offsets): the
-//     register-staged form below.
+//   * gemm2_kernel: the register-staged form below, for bf16 launches where
+//     its reads share the L2 better (gemm2_bf16_regs) and operands past the
+//     pipelines' 32-bit buffer offsets.
 // The pipelines also hold copies that compute only the first 16 / 32
 // positions of a tile, taken by tiles with no more (an expert's last or
 // only tile): the matrix-core work of empty column tiles is skipped, and an
@@ -76,8 +77,17 @@ struct ARegs {
 // remaining slabs.  (The 1-D grid is a multiple of 8 and at least
 // 8 * per_xcd, so every item below n_items has exactly one workgroup.)
 // Returns false for a workgroup without an item.
-// slabs per group: all of them unless one expert's weights pass 4 MiB
-int slab_group(int n_slabs, int64_t expert_bytes) { return expert_bytes > (4 << 20) ? min(4, n_slabs) : n_slabs; }
+// slabs per group: all of them unless one expert's weights pass 4 MiB; two
+// for bf16 experts past 64 MiB, of whose slabs (2 MiB and more each) four
+// leave the L2 before an expert's next tile reads them.  Measured, bf16, us
+// per layer, four -> two: Mixtral-8x7B (224 and 112 MiB) T = 500 / 1000 /
+// 2048 878 / 1265 / 2183 -> 837 / 1180 / 1996, T = 200 546 -> 549; H = I =
+// 4096, 8 experts (64 and 32 MiB; its 8 groups of four are one per XCD)
+// T = 300 / 500 204 / 262 against 210 / 268.
+int slab_group(int wf, int n_slabs, int64_t expert_bytes) {
+  if (expert_bytes <= (4 << 20)) return n_slabs;
+  return min(wf == WF_BF16 && expert_bytes > (64 << 20) ? 2 : 4, n_slabs);
+}
 
 struct TileItem {
   int expert, row0, rows, slab;
@@ -823,7 +833,8 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
 // registers (one vector offset serves all eight loads; with a vector offset
 // per row the nt copy of the full tile spilled).  Bound by the weight stream
 // from HBM until experts hold a few tiles, then by waits; the register-staged
-// gemm2_kernel kept one eight-wave workgroup per CU and no short-tile copies.
+// gemm2_kernel keeps one eight-wave workgroup per CU and has no short-tile
+// copies (launch_gemm2 still takes it for few large experts: gemm2_bf16_regs).
 // Measured, gemm2_kernel -> this (Qwen3 bf16, us per layer): T = 200 / 700 /
 // 1000 / 2000 / 4096 230 / 275 / 282 / 375 / 606 -> 207 / 249 / 277 / 356 /
 // 535; the full tile's nt copy (an expert's only tile of 49 - 64 positions)
@@ -1393,8 +1404,8 @@ static double gemm2_expected_tiles(const GemmArgs& a, int max_tiles) {
   return n < kBM ? experts * (1.0 + (n - 50.0) / (2.0 * (kBM - 50.0))) : a.num_rows / (double)kBM + 0.5 * experts;
 }
 
-// Eight waves per workgroup instead of four (the results are the same bit for
-// bit).  int4: while the launch has at most one (tile, slab) item per CU -- a
+// int4 on eight waves per workgroup instead of four (the results are the same
+// bit for bit): while the launch has at most one (tile, slab) item per CU -- a
 // lone four-wave workgroup leaves its SIMDs one wave each.  Measured, us, four
 // waves against eight, weights from HBM: gate_up H = 2048 I = 768, 16 experts,
 // 96 / 144 / 240 items 24.4 / 28.6 / 29.4 against 20.2 / 23.7 / 24.4; H = I =
@@ -1405,8 +1416,34 @@ static double gemm2_expected_tiles(const GemmArgs& a, int max_tiles) {
 // 72.6.
 constexpr double kGemm2Cus = 256.0;
 
-static bool gemm2_eight_waves(const GemmArgs& a, int wf, int n_slabs, int max_tiles) {
-  return wf == WF_I4 && n_slabs * gemm2_expected_tiles(a, max_tiles) <= kGemm2Cus;
+static bool gemm2_i4_eight_waves(const GemmArgs& a, int n_slabs, int max_tiles) {
+  return n_slabs * gemm2_expected_tiles(a, max_tiles) <= kGemm2Cus;
+}
+
+// bf16 weights on the register-staged gemm2_kernel instead of the pipeline
+// (the results are the same bit for bit).  Its 128-wide steps read a row
+// block 4 KiB at a time, and its eight waves a CU (one workgroup) keep an
+// expert's tiles close enough to share a slab's reads in the L2: Mixtral-8x7B
+// gate_up at T = 300 fetches 7 % more than its weights, the pipeline 26 %.
+//   * down: few items of many K steps.  Pipeline -> this, us per layer:
+//     Mixtral-8x7B (K = 14336) T = 100 / 300 / 500 / 1000 516 / 634 / 837 /
+//     1180 -> 506 / 614 / 818 / 1168, T = 2048 1996 -> 2024; H = I = 4096, 8
+//     experts, T = 300 / 400 204 / 209 -> 199 / 202, T = 500 (314 items) 262
+//     -> 265; at K = 2048 never faster.
+//   * gate_up: once experts hold a second tile (before, the nt copies of the
+//     pipeline win: Mixtral-8x7B T = 200 / 230 546 / 565 against 560 / 573),
+//     for launches of about one item per CU (16 experts, H = 2048 I = 768,
+//     T = 600 / 1000 65.1 / 72.0 -> 62.8 / 69.6; 400 items of 8 experts, H =
+//     I = 2048, T = 700 94.7 against 98.1) and for large experts up to four
+//     tiles (Mixtral-8x7B T = 300 / 400 646 / 624 -> 618 / 605, T = 800 985
+//     -> 959, H = I = 4096 T = 300 / 700 / 1000 204 / 289 / 366 -> 197 / 283 /
+//     362, T = 2048 593 against 618; 60 experts of 11 MiB T = 800 / 1200 197
+//     / 264 against 212 / 265).
+static bool gemm2_bf16_regs(const GemmArgs& a, int phase, int n_slabs, int max_tiles) {
+  const double items = n_slabs * gemm2_expected_tiles(a, max_tiles);
+  if (phase == PHASE_DOWN) return a.K >= 4096 && 15.0 * items <= a.K;
+  const double avg = a.num_rows / (a.n_tiles ? (double)(max_tiles - a.num_rows / kBM) : 1.0);
+  return avg >= 60.0 && (items <= 1.0625 * kGemm2Cus || (a.w_expert_bytes > (16 << 20) && avg < 256.0));
 }
 
 hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hipStream_t stream,
@@ -1419,7 +1456,7 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
     return hipErrorInvalidValue;
   const int n_slabs = phase == PHASE_GATE_UP ? a.I / 128 : a.N / 256 * kp;
   const int64_t items = (int64_t)n_slabs * max_tiles;
-  const int sg = slab_group(n_slabs, a.w_expert_bytes);
+  const int sg = slab_group(wf, n_slabs, a.w_expert_bytes);
   dim3 grid((unsigned)((items + kXcds - 1) / kXcds * kXcds)), block(64 * gemm2_waves(wf));
 #define NKT_G2(W)                                                                                          \
   case W:                                                                                                  \
@@ -1437,7 +1474,7 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
       launch_timed(gemm2_i8_kernel<PHASE_DOWN, false>, grid, block, 0, stream, tm, a, n_slabs, sg);
     return hipGetLastError();
   }
-  if (gemm2_bf16_pipeline(a, wf)) {
+  if (gemm2_bf16_pipeline(a, wf) && !gemm2_bf16_regs(a, phase, n_slabs, max_tiles)) {
     if (phase == PHASE_GATE_UP)
       launch_timed(gemm2_bf16_kernel<PHASE_GATE_UP>, grid, dim3(256), 0, stream, tm, a, n_slabs, sg);
     else
@@ -1445,7 +1482,7 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
     return hipGetLastError();
   }
   if (gemm2_i4_pipeline(a, wf)) {
-    const bool w8 = gemm2_eight_waves(a, wf, n_slabs, max_tiles);
+    const bool w8 = gemm2_i4_eight_waves(a, n_slabs, max_tiles);
     block = dim3(w8 ? 512 : 256);
     if (phase == PHASE_GATE_UP && w8)
       launch_timed(gemm2_i4_kernel<PHASE_GATE_UP, 8>, grid, block, 0, stream, tm, a, n_slabs, sg);

@@ -48,3 +48,21 @@ def test_int4_rows_same_bits_in_every_batch(gpu_device):
         part = native.forward(x[:T].contiguous(), logits[:T].contiguous())
         torch.cuda.synchronize()
         assert torch.equal(full[:T], part), f"T = {T}"
+
+
+def test_bf16_rows_same_bits_in_every_batch(gpu_device):
+    """A bf16 prefill row does not depend on the batch either: experts of 20
+    MiB whose gate_up leaves the stage pipeline for the register-staged form
+    from 60 to 255 positions per expert (T = 300, 1000), and whose down (K =
+    4096, 5 slabs) leaves it up to 273 (tile, slab) items (T = 2200 above)."""
+    cfg = replace(CONFIGS["qwen3_int4"], name="few_experts_bf16", H=1280, I=4096, E=8, k=2, wfmt="bf16")
+    layer = build_layer(cfg, device="cuda")
+    native = native_layer(layer, torch.device("cuda"))
+    x, logits = build_inputs(layer, 2200, seed=5, device="cuda")
+    full = native.forward(x, logits).clone()
+    compare(full[:97].float().cpu().numpy(), oracle_forward(layer, x[:97], logits[:97]), cfg)
+    for T in (97, 300, 1000, 1500):
+        assert not cfg.decode_form(T)
+        part = native.forward(x[:T].contiguous(), logits[:T].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(full[:T], part), f"T = {T}"
