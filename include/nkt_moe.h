@@ -104,7 +104,9 @@ extern "C" {
 /* Create a handle for one layer shape.
  * Replaces the construction of HybridMoE's expert state
  * (nano_ktrans/layers/hybrid_moe.py:55-290).  shared_inter = 0: no shared
- * expert.  max_tokens bounds num_tokens of every later call.  Returns NULL on
+ * expert.  max_tokens bounds num_tokens of every later call.  Refused: one
+ * expert's (or the shared expert's) gate_up of 4 GiB or more in the bf16, int8
+ * and int4 formats, and activations of 4 GiB or more.  Returns NULL on
  * failure. */
 void* nkt_moe_create(int num_experts, int top_k, int hidden_size, int moe_intermediate_size,
                      int shared_intermediate_size, int weight_format, int act_dtype,

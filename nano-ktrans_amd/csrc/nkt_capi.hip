@@ -1041,6 +1041,18 @@ void* nkt_moe_create(int num_experts, int top_k, int hidden_size, int moe_interm
       return nullptr;
     }
   }
+  if (weight_format != NKT_WEIGHT_F32) {
+    // and one expert's projection likewise (the fp32 form uses 64-bit
+    // addresses); gate_up is the larger of its two
+    const int64_t imax = shared_intermediate_size > moe_intermediate_size ? shared_intermediate_size
+                                                                          : moe_intermediate_size;
+    const int64_t codes = 2 * imax * hidden_size * bytes_per_weight_x2(weight_format) / 2;
+    if (codes >= ((int64_t)1 << 32)) {
+      set_err(err, err_len, "intermediate size %lld x hidden_size %d: one expert's gate_up would reach 4 GiB",
+              (long long)imax, hidden_size);
+      return nullptr;
+    }
+  }
   Handle* h = new (std::nothrow) Handle();
   if (!h) {
     set_err(err, err_len, "out of host memory");

@@ -16,8 +16,9 @@
 //   * gemm2_bf16_kernel (bf16): the int8 pipeline's form, two weight blocks
 //     per row tile and stage;
 //   * gemm2_kernel: the register-staged form below, for bf16 launches where
-//     its reads share the L2 better (gemm2_bf16_regs) and operands past the
-//     pipelines' 32-bit buffer offsets.
+//     its reads share the L2 better (gemm2_bf16_regs) and experts of 2 GiB
+//     and more.  (All address one expert's projection with 32-bit offsets;
+//     a handle holds none of 4 GiB or more.)
 // The pipelines also hold copies that compute only the first 16 / 32
 // positions of a tile, taken by tiles with no more (an expert's last or
 // only tile): the matrix-core work of empty column tiles is skipped, and an
@@ -53,14 +54,6 @@ constexpr int kBM = 64;           // positions per tile
 constexpr int kCT = kBM / 16;     // 16-position MFMA column tiles
 
 constexpr int kXcds = 8;          // MI355X: accelerator complex dies, each with its own L2
-
-template <int WF, int kRT>
-struct ARegs {
-  static constexpr int NBLK = 128 / block_k(WF);
-  u32x4 w[kRT][NBLK];
-  u32x2 s[kRT];
-};
-
 
 }  // namespace
 
@@ -394,46 +387,42 @@ __device__ __forceinline__ void gemm2_epilogue(const GemmArgs& a, f32x4 (&acc)[1
   }
 }
 
-template <int WF, int PHASE, int kWaves>
-__global__ void __launch_bounds__(64 * kWaves, 2) gemm2_kernel(GemmArgs a, int n_slabs, int sg) {
-  constexpr int kRT = 16 / kWaves;  // 16-row weight tiles per wave
-  constexpr int NBLK = 128 / block_k(WF);
-  // two separate LDS objects (not one array) so the compiler can tell a
-  // direct-to-LDS load into one buffer from reads of the other
+// bf16 weights, register-staged (launch_gemm2's rule says when): eight waves of
+// two row tiles each, which halves the weight registers a wave double-buffers
+// against four waves of four.
+template <int PHASE>
+__global__ void __launch_bounds__(512, 2) gemm2_kernel(GemmArgs a, int n_slabs, int sg) {
+  constexpr int kWaves = 8;
+  constexpr int kRT = 16 / kWaves;              // 16-row weight tiles per wave
+  constexpr int NBLK = 128 / block_k(WF_BF16);  // 1 KiB weight blocks per row tile and 128-wide step
+  // two separate LDS objects (not one array) so the compiler can tell writes
+  // of one buffer from reads of the other
   __shared__ __attribute__((aligned(1024))) uint8_t bt0[kBM * 256];
   __shared__ __attribute__((aligned(1024))) uint8_t bt1[kBM * 256];
-  __shared__ float xsl0[256];  // int4: group sums of the tile rows (each wave loads all; [0, kBM) used)
-  __shared__ float xsl1[256];
   __shared__ int srcl[kBM];
   __shared__ int orow_l[kBM];
   __shared__ float hpart[kWaves][kBM];
-  __shared__ float xtot_l[kBM];
 
   TileItem it;
   if (!gemm2_item(a, n_slabs, sg, it)) return;
-  const int expert = it.expert, row0 = it.row0, rows = it.rows, slab = it.slab;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int G = a.K / 128;
-  const int NKB = a.K / block_k(WF);
   gemm2_sources(a, it, srcl, orow_l);
   __syncthreads();
 
   // ---- this wave's weight rows ------------------------------------------
-  const uint8_t* wexp = a.w + (int64_t)expert * a.w_expert_bytes;
-  const uint16_t* sexp = a.scales + (int64_t)expert * a.s_expert_elems;
+  const uint8_t* wexp = a.w + (int64_t)it.expert * a.w_expert_bytes;
   int wrow[kRT];
-  uint32_t woff[kRT], soff[kRT];
+  uint32_t woff[kRT];
 #pragma unroll
   for (int r = 0; r < kRT; ++r) {
     if (PHASE == PHASE_GATE_UP)
-      wrow[r] = (r < kRT / 2 ? 0 : a.I) + slab * 128 + wave * (128 / kWaves) + (r % (kRT / 2)) * 16;
+      wrow[r] = (r < kRT / 2 ? 0 : a.I) + it.slab * 128 + wave * (128 / kWaves) + (r % (kRT / 2)) * 16;
     else
-      wrow[r] = slab * 256 + wave * (256 / kWaves) + r * 16;
-    const uint32_t rb = (uint32_t)(wrow[r] >> 4);
-    woff[r] = rb * (uint32_t)NKB * 1024u + (uint32_t)lane * 16u;
-    soff[r] = rb * (uint32_t)G * 16u + 4u * (uint32_t)(lane >> 4);
+      wrow[r] = it.slab * 256 + wave * (256 / kWaves) + r * 16;
+    woff[r] = (uint32_t)(wrow[r] >> 4) * (uint32_t)(G * NBLK) * 1024u + (uint32_t)lane * 16u;
   }
 
   // ---- token-tile staging: 16 / kWaves x 16 B per thread per group --------
@@ -447,27 +436,23 @@ __global__ void __launch_bounds__(64 * kWaves, 2) gemm2_kernel(GemmArgs a, int n
 #pragma unroll
   for (int i = 0; i < NST; ++i)
     boff[i] = (uint32_t)srcl[i * 4 * kWaves + (tid >> 4)] * (uint32_t)a.K * 2u + (tid & 15) * 16u;
-  const int xs_src = tid < kBM ? srcl[tid] : 0;
-  auto load_b = [&](u32x4(&st)[NST], float& xsv, int g) {
+  auto load_b = [&](u32x4(&st)[NST], int g) {
 #pragma unroll
     for (int i = 0; i < NST; ++i) st[i] = *(const u32x4*)(inb + (boff[i] + (uint32_t)g * 256u));
-    if (WF == WF_I4) xsv = a.xsum[(int64_t)xs_src * G + g];
   };
-  auto store_b = [&](const u32x4(&st)[NST], float xsv, uint8_t* bt, float* xsl) {
+  auto store_b = [&](const u32x4(&st)[NST], uint8_t* bt) {
 #pragma unroll
     for (int i = 0; i < NST; ++i) {
       const int r = i * 4 * kWaves + (tid >> 4);
       *(u32x4*)(bt + r * 256 + (((tid & 15) ^ (r & 15)) * 16)) = st[i];
     }
-    if (WF == WF_I4 && tid < kBM) xsl[tid] = xsv;
   };
-  auto load_a = [&](ARegs<WF, kRT>& A, int g) {
+  typedef u32x4 ARegs[kRT][NBLK];
+  auto load_a = [&](ARegs& A, int g) {
 #pragma unroll
-    for (int r = 0; r < kRT; ++r) {
+    for (int r = 0; r < kRT; ++r)
 #pragma unroll
-      for (int i = 0; i < NBLK; ++i) A.w[r][i] = *(const u32x4*)(wexp + (woff[r] + (uint32_t)(g * NBLK + i) * 1024u));
-      if (WF == WF_I4) A.s[r] = *(const u32x2*)(sexp + (soff[r] + (uint32_t)g * 16u));
-    }
+      for (int i = 0; i < NBLK; ++i) A[r][i] = *(const u32x4*)(wexp + (woff[r] + (uint32_t)(g * NBLK + i) * 1024u));
   };
 
   f32x4 acc[kRT][kCT];
@@ -476,59 +461,26 @@ __global__ void __launch_bounds__(64 * kWaves, 2) gemm2_kernel(GemmArgs a, int n
 #pragma unroll
     for (int c = 0; c < kCT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  auto compute = [&](const ARegs<WF, kRT>& A, const uint8_t* bb, const float* xsl) {
-    if (WF == WF_I4) {
-      // per-group scale: each (row tile, column tile) sums its 4 steps in a
-      // temporary that starts at the offset correction, then is scaled in
-      u32x4 ad[kRT][4];
-      f32x4 sc[kRT];
+  // one 32-wide K step at a time: the wave's A fragments and 4 B fragments
+  // feed independent accumulators; the next step's B fragments load while
+  // this step's MFMAs run (two fragment sets live, pinned by scheduling
+  // barriers so the compiler does not hoist more)
+  auto compute = [&](const ARegs& A, const uint8_t* bb) {
+    u32x4 bf[2][kCT];
+    auto read_b = [&](u32x4(&f)[kCT], int s) {
 #pragma unroll
-      for (int r = 0; r < kRT; ++r) {
-        sc[r] = bf16x4_to_f32(A.s[r]);
+      for (int c = 0; c < kCT; ++c)
+        f[c] = *(const u32x4*)(bb + (c * 16 + (lane & 15)) * 256 + (((4 * s + (lane >> 4)) ^ (lane & 15)) * 16));
+    };
+    read_b(bf[0], 0);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) ad[r][s] = dq_i4(A.w[r][0][s]);
-      }
+    for (int s = 0; s < 4; ++s) {
+      if (s + 1 < 4) read_b(bf[(s + 1) & 1], s + 1);
 #pragma unroll
-      for (int c = 0; c < kCT; ++c) {
-        const int prow = c * 16 + (lane & 15);
-        u32x4 bf[4];
+      for (int c = 0; c < kCT; ++c)
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
-          bf[s] = *(const u32x4*)(bb + prow * 256 + (((4 * s + (lane >> 4)) ^ (lane & 15)) * 16));
-        const float cv = -136.0f * xsl[prow];
-#pragma unroll
-        for (int r = 0; r < kRT; ++r) {
-          f32x4 tmp = f32x4{cv, cv, cv, cv};
-#pragma unroll
-          for (int s = 0; s < 4; ++s) tmp = mfma_bf16(ad[r][s], bf[s], tmp);
-          acc[r][c] += sc[r] * tmp;
-        }
-      }
-    } else {
-      // one 32-wide K step at a time: 4 dequantised A fragments and 8 B
-      // fragments feed 32 independent accumulators; the next step's B
-      // fragments load while this step's MFMAs run (two fragment sets live,
-      // pinned by scheduling barriers so the compiler does not hoist more)
-      u32x4 bf[2][kCT];
-      auto read_b = [&](u32x4(&f)[kCT], int s) {
-#pragma unroll
-        for (int c = 0; c < kCT; ++c)
-          f[c] = *(const u32x4*)(bb + (c * 16 + (lane & 15)) * 256 + (((4 * s + (lane >> 4)) ^ (lane & 15)) * 16));
-      };
-      read_b(bf[0], 0);
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        if (s + 1 < 4) read_b(bf[(s + 1) & 1], s + 1);
-        u32x4 ad[kRT];
-#pragma unroll
-        for (int r = 0; r < kRT; ++r)
-          ad[r] = (WF == WF_I8) ? dq_i8(A.w[r][s >> 1][2 * (s & 1)], A.w[r][s >> 1][2 * (s & 1) + 1]) : A.w[r][s];
-#pragma unroll
-        for (int c = 0; c < kCT; ++c)
-#pragma unroll
-          for (int r = 0; r < kRT; ++r) acc[r][c] = mfma_bf16(ad[r], bf[s & 1][c], acc[r][c]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+        for (int r = 0; r < kRT; ++r) acc[r][c] = mfma_bf16(A[r][s], bf[s & 1][c], acc[r][c]);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -539,34 +491,33 @@ __global__ void __launch_bounds__(64 * kWaves, 2) gemm2_kernel(GemmArgs a, int n
   // and the workgroup meets at an LDS-only barrier (the weight loads stay in
   // flight).  The loads are pinned above the MFMAs (the scheduler would sink
   // them to their use); past the last group they repeat it (no load behind a
-  // branch).  The second workgroup on the CU computes while this one waits.
-  ARegs<WF, kRT> A0, A1;
+  // branch).
+  ARegs A0, A1;
   u32x4 st[NST];
-  float xsv = 0.f;
-  load_b(st, xsv, 0);
+  load_b(st, 0);
   load_a(A0, 0);
-  store_b(st, xsv, bt0, xsl0);
+  store_b(st, bt0);
   __syncthreads();
   for (int g = 0; g < G; g += 2) {
-    load_b(st, xsv, min(g + 1, G - 1));
+    load_b(st, min(g + 1, G - 1));
     load_a(A1, min(g + 1, G - 1));
     __builtin_amdgcn_sched_barrier(0);
-    compute(A0, bt0, xsl0);
+    compute(A0, bt0);
     if (g + 1 >= G) break;
-    store_b(st, xsv, bt1, xsl1);
+    store_b(st, bt1);
     lds_barrier();
-    load_b(st, xsv, min(g + 2, G - 1));
+    load_b(st, min(g + 2, G - 1));
     load_a(A0, min(g + 2, G - 1));
     __builtin_amdgcn_sched_barrier(0);
-    compute(A1, bt1, xsl1);
+    compute(A1, bt1);
     if (g + 2 >= G) break;
-    store_b(st, xsv, bt0, xsl0);
+    store_b(st, bt0);
     lds_barrier();
   }
   __syncthreads();
 
-  gemm2_epilogue<WF, PHASE, kWaves>(a, acc, srcl, orow_l, hpart, xtot_l, xtot_l, wrow, sexp, row0, rows, slab,
-                                    nullptr, WF == WF_I4 && PHASE == PHASE_GATE_UP ? bt0 : nullptr);
+  gemm2_epilogue<WF_BF16, PHASE, kWaves>(a, acc, srcl, orow_l, hpart, nullptr, nullptr, wrow, nullptr, it.row0, it.rows,
+                                         it.slab);
 }
 
 // ---------------------------------------------------------------------------
@@ -1385,13 +1336,6 @@ hipError_t launch_group_sums(const void* x, int rows, int K, float* out, hipStre
   return hipGetLastError();
 }
 
-// Waves per workgroup: int8 keeps 4 waves of 4 row tiles (its dequantised
-// fragments feed 4 column tiles each and its loop fits two workgroups per CU
-// without spills); bf16 and int4 take 8 waves of 2 row tiles, which halves
-// the weight registers a wave double-buffers (bf16 blocks hold 32 columns,
-// int4 adds per-group scale temporaries) and removes their spills.
-constexpr int gemm2_waves(int wf) { return wf == WF_I8 ? 4 : 8; }
-
 // Tiles the launch can expect: exact for a dense launch; for a tile list
 // (max_tiles is its upper bound, all full tiles and one more per expert) from
 // the mean positions per expert -- one tile each up to 50 (at 64 half of the
@@ -1457,14 +1401,7 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
   const int n_slabs = phase == PHASE_GATE_UP ? a.I / 128 : a.N / 256 * kp;
   const int64_t items = (int64_t)n_slabs * max_tiles;
   const int sg = slab_group(wf, n_slabs, a.w_expert_bytes);
-  dim3 grid((unsigned)((items + kXcds - 1) / kXcds * kXcds)), block(64 * gemm2_waves(wf));
-#define NKT_G2(W)                                                                                          \
-  case W:                                                                                                  \
-    if (phase == PHASE_GATE_UP)                                                                            \
-      launch_timed(gemm2_kernel<W, PHASE_GATE_UP, gemm2_waves(W)>, grid, block, 0, stream, tm, a, n_slabs, sg); \
-    else                                                                                                   \
-      launch_timed(gemm2_kernel<W, PHASE_DOWN, gemm2_waves(W)>, grid, block, 0, stream, tm, a, n_slabs, sg);    \
-    break;
+  dim3 grid((unsigned)((items + kXcds - 1) / kXcds * kXcds)), block(256);
   if (gemm2_i8_pipeline(a, wf)) {
     if (phase == PHASE_GATE_UP && a.xinv)
       launch_timed(gemm2_i8_kernel<PHASE_GATE_UP, true>, grid, block, 0, stream, tm, a, n_slabs, sg);
@@ -1474,11 +1411,19 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
       launch_timed(gemm2_i8_kernel<PHASE_DOWN, false>, grid, block, 0, stream, tm, a, n_slabs, sg);
     return hipGetLastError();
   }
-  if (gemm2_bf16_pipeline(a, wf) && !gemm2_bf16_regs(a, phase, n_slabs, max_tiles)) {
+  if (wf == WF_BF16 && (!gemm2_bf16_pipeline(a, wf) || gemm2_bf16_regs(a, phase, n_slabs, max_tiles))) {
+    block = dim3(512);
     if (phase == PHASE_GATE_UP)
-      launch_timed(gemm2_bf16_kernel<PHASE_GATE_UP>, grid, dim3(256), 0, stream, tm, a, n_slabs, sg);
+      launch_timed(gemm2_kernel<PHASE_GATE_UP>, grid, block, 0, stream, tm, a, n_slabs, sg);
     else
-      launch_timed(gemm2_bf16_kernel<PHASE_DOWN>, grid, dim3(256), 0, stream, tm, a, n_slabs, sg);
+      launch_timed(gemm2_kernel<PHASE_DOWN>, grid, block, 0, stream, tm, a, n_slabs, sg);
+    return hipGetLastError();
+  }
+  if (wf == WF_BF16) {
+    if (phase == PHASE_GATE_UP)
+      launch_timed(gemm2_bf16_kernel<PHASE_GATE_UP>, grid, block, 0, stream, tm, a, n_slabs, sg);
+    else
+      launch_timed(gemm2_bf16_kernel<PHASE_DOWN>, grid, block, 0, stream, tm, a, n_slabs, sg);
     return hipGetLastError();
   }
   if (gemm2_i4_pipeline(a, wf)) {
@@ -1494,14 +1439,7 @@ hipError_t launch_gemm2(const GemmArgs& a, int wf, int phase, int max_tiles, hip
       launch_timed(gemm2_i4_kernel<PHASE_DOWN, 4>, grid, block, 0, stream, tm, a, n_slabs, sg);
     return hipGetLastError();
   }
-  switch (wf) {
-    NKT_G2(WF_BF16)
-    NKT_G2(WF_I4)
-    default:
-      return hipErrorInvalidValue;
-  }
-#undef NKT_G2
-  return hipGetLastError();
+  return hipErrorInvalidValue;  // no such handle: an expert's projection stays under 4 GiB
 }
 
 }  // namespace nkt

@@ -49,6 +49,25 @@ def test_create_rejects_bad_arguments(kw, msg):
     assert msg in err
 
 
+@pytest.mark.parametrize("wf,k", [(N.WEIGHT_BF16, 2), (N.WEIGHT_INT8_PC, 1), (N.WEIGHT_INT4_G128, 0.5)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_create_rejects_experts_past_32_bit_offsets(wf, k, shared):
+    """The expert kernels address one expert's gate_up (2 I x H weights of k
+    bytes) with 32-bit offsets: one of 4 GiB is refused, 128 columns less are
+    not; fp32 layers use 64-bit addresses and take both."""
+    H = 4096
+    I = int((1 << 32) / (2 * H * k))
+    dims = (lambda n: dict(I=128, Is=n)) if shared else (lambda n: dict(I=n))
+    h, err = _create(H=H, wf=wf, act=N.DTYPE_BF16, max_tokens=1, **dims(I))
+    assert not h and "4 GiB" in err
+    h, err = _create(H=H, wf=wf, act=N.DTYPE_BF16, max_tokens=1, **dims(I - 128))
+    assert h, err
+    N.lib().nkt_moe_destroy(h)
+    h, err = _create(H=H, max_tokens=1, **dims(I))
+    assert h, err
+    N.lib().nkt_moe_destroy(h)
+
+
 def test_weight_and_workspace_sizes():
     lib = N.lib()
     E, k, H, I, Is = 60, 4, 2048, 1408, 5632

@@ -9,7 +9,7 @@ from dataclasses import replace
 import pytest
 import torch
 
-from moe_cases import CONFIGS, build_inputs, build_layer, compare, native_layer, oracle_forward
+from moe_cases import CONFIGS, Layer, build_inputs, build_layer, compare, native_layer, oracle_forward
 
 pytestmark = pytest.mark.gpu
 
@@ -66,3 +66,27 @@ def test_bf16_rows_same_bits_in_every_batch(gpu_device):
         part = native.forward(x[:T].contiguous(), logits[:T].contiguous())
         torch.cuda.synchronize()
         assert torch.equal(full[:T], part), f"T = {T}"
+
+
+def test_bf16_expert_past_2_gib(gpu_device):
+    """One expert whose gate_up takes 2 GiB (the up rows past 1 GiB, the last
+    ones close to 2): gemm2_kernel's range, against the same products in
+    fp32 on the same bf16 values.  Tolerance as in moe_cases.compare."""
+    H, I, T = 4096, 131072, 70
+    cfg = replace(CONFIGS["qwen3_int4"], name="bf16_2gib", H=H, I=I, E=1, k=1, wfmt="bf16")
+    g = torch.Generator(device="cuda").manual_seed(9)
+
+    def randn(n, k, std):
+        return torch.empty(n, k, dtype=torch.bfloat16, device="cuda").normal_(0, std, generator=g)
+
+    native = native_layer(Layer(cfg, torch.zeros(1, H), []), torch.device("cuda"), max_tokens=T)
+    gate, up, down = randn(I, H, 0.02), randn(I, H, 0.02), randn(H, I, 0.002)  # y of std about 0.6
+    native.load_expert(0, gate, up, down)
+    x = torch.randn(T, H, device="cuda", generator=g).to(torch.bfloat16)
+    out = native.forward(x, torch.zeros(T, 1, dtype=torch.bfloat16, device="cuda"))
+    torch.cuda.synchronize()
+    ref = torch.zeros(T, H, device="cuda")
+    for i in range(0, I, 16384):
+        a, b = x.float() @ gate[i:i + 16384].float().T, x.float() @ up[i:i + 16384].float().T
+        ref += (torch.nn.functional.silu(a) * b) @ down[:, i:i + 16384].float().T
+    compare(out.float().cpu().numpy(), ref.cpu().numpy(), cfg)
