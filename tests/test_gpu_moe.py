@@ -111,11 +111,10 @@ def test_qwen3_int4_full(gpu_device, T):
 @pytest.mark.parametrize("name,E,T", [("qwen3_int4", None, 300), ("qwen3_int4", 32, 90),
                                       ("qwen3_int8", 32, 40), ("qwen3_int8", 32, 100)])
 def test_prefill_short_tile_copies(gpu_device, name, E, T):
-    """Prefill tiles of at most 16 / 32 positions (an expert's last or only
-    tile) run pipeline copies over their first 1 / 2 column tiles: int8
-    always (the Zipf-skewed qwen3_int8 routing gives tiles of every size),
-    int4 where the experts average at most 24 positions (T k <= 24 E: 18.75
-    and 22.5 per expert here, tiles of 5 - 40 positions)."""
+    """Prefill tiles of at most 16 / 32 / 48 positions (an expert's last or
+    only tile) run pipeline copies over their first 1 / 2 / 3 column tiles
+    (the Zipf-skewed qwen3_int8 routing gives tiles of every size, the int4
+    batches, 18.75 and 22.5 positions per expert, tiles of 5 - 40)."""
     announce(f"forward {name} E={E} T={T} (short prefill tiles)")
     layer, native = _layer(name, E=E)
     assert not layer.cfg.decode_form(T)
@@ -459,7 +458,8 @@ def _check_rows_and_prefix(layer, native, T, prefix, seed):
     """The full batch's routing and permutation bit-exact; >= 97 spread rows
     against the oracle; rows [0, prefix) bit-identical to a batch of prefix
     tokens (the same prefill regime: every output element sums over K in the
-    same order whatever the tile)."""
+    same order whatever the tile, the waves per workgroup or, for bf16, the
+    kernel; int8's shared expert has a regime of its own, by its K parts)."""
     cfg = layer.cfg
     x, logits = build_inputs(layer, T, seed=seed, device="cuda")
     out = native.forward(x, logits).clone()

@@ -1,9 +1,17 @@
 """Prefill-form expert GEMMs at the edges of their K pipelines and token tiles.
 
-Two experts that every token picks, so each holds T positions: T around the
-16-position column tiles and the 64-position tiles, and H / I so that gate_up
-and down end in every remainder of the unrolled stage loop (1 .. 8 stages of
-128).  Tolerance as in moe_cases.compare (bf16 outputs)."""
+Two experts that every token picks, so each holds T positions, T around the
+16-position column tiles and the 64-position tiles.  The pipelines' loops take
+six stages a round and up to five after it: int4 runs H / 128 stages in gate_up
+(H is a multiple of 256, so remainders 0, 2 and 4) and I / 128 in down
+(remainders 0 .. 5, with and without a full round before them); int8 and bf16
+run H / 64 and I / 64, both even (0, 2, 4).
+
+Small batches are checked against the oracle (tolerance as in
+moe_cases.compare, bf16 outputs): int4 there runs eight waves per workgroup,
+bf16's gate_up the register-staged kernel from 60 positions on.  Large batches, where
+int4 runs four waves and bf16 its pipeline, are checked bit for bit against
+the small ones."""
 from dataclasses import replace
 
 import pytest
@@ -13,8 +21,9 @@ from moe_cases import CONFIGS, Layer, build_inputs, build_layer, compare, native
 
 pytestmark = pytest.mark.gpu
 
-# (H, I): gate_up runs H / 128 stages, down I / 128
-SHAPES = [(256, 128), (512, 384), (768, 640), (1024, 256), (1280, 896), (256, 512)]
+# (H, I) in 128-wide stages: 2/1, 4/3, 6/5, 8/2, 10/7, 2/4, 12/6, 2/11, 4/8, 6/9, 2/10
+SHAPES = [(256, 128), (512, 384), (768, 640), (1024, 256), (1280, 896), (256, 512), (1536, 768), (256, 1408),
+          (512, 1024), (768, 1152), (256, 1280)]
 
 
 @pytest.mark.parametrize("wfmt", ["int4_g128", "bf16", "int8_per_channel"])
@@ -23,12 +32,35 @@ def test_stage_and_tile_remainders(gpu_device, wfmt, H, I):
     cfg = replace(CONFIGS["qwen3_int4"], name=f"stages_{wfmt}", H=H, I=I, E=2, k=2, wfmt=wfmt)
     layer = build_layer(cfg, device="cuda")
     native = native_layer(layer, torch.device("cuda"))
-    for T in (13, 17, 33, 49, 64, 65, 130):
+    # last tiles of 13 .. 64 positions alone, of 1, 2, 16, 26, 41 and 56 after a full one
+    for T in (13, 17, 33, 49, 64, 65, 130, 80, 90, 105, 120):
         x, logits = build_inputs(layer, T, seed=T, device="cuda")
         out = native.forward(x, logits)
         torch.cuda.synchronize()
         ref = oracle_forward(layer, x, logits)
         compare(out.float().cpu().numpy(), ref, cfg)
+
+
+@pytest.mark.parametrize("wfmt", ["int4_g128", "bf16", "int8_per_channel"])
+@pytest.mark.parametrize("H,I", SHAPES)
+def test_stage_and_tile_remainders_in_large_batches(gpu_device, wfmt, H, I):
+    """Batches of more than 272 (tile, slab) items in either projection and
+    more than 256 positions per expert whose last tile holds r: its rows, and
+    the first full tile's, have the bits of a batch of those tokens alone."""
+    cfg = replace(CONFIGS["qwen3_int4"], name=f"stages_{wfmt}", H=H, I=I, E=2, k=2, wfmt=wfmt)
+    layer = build_layer(cfg, device="cuda")
+    native = native_layer(layer, torch.device("cuda"), max_tokens=9000)
+    slabs = min(I // 128, H // 256)
+    full = max(5, (272 // slabs) // 2 + 1)  # full tiles of each expert: slabs * (2 full + 1) > 272
+    x, logits = build_inputs(layer, 64 * full + 64, seed=7, device="cuda")
+    first = native.forward(x[:64].contiguous(), logits[:64].contiguous()).clone()
+    for r in (13, 26, 41, 57, 64):
+        T = 64 * full + r
+        out = native.forward(x[:T].contiguous(), logits[:T].contiguous()).clone()
+        alone = native.forward(x[64 * full:T].contiguous(), logits[64 * full:T].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(out[64 * full:], alone), f"last tile of {r}"
+        assert torch.equal(out[:64], first), f"first tile, r = {r}"
 
 
 def test_int4_rows_same_bits_in_every_batch(gpu_device):
