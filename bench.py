@@ -29,16 +29,17 @@ Printed JSON fields beyond the standard ones:
                  multiply-adds as one dense [T k, N, K] GEMM) for the MFMA bound
   cpu_baseline   the reference CPU expert loop (oracle/cpu_loop.py, a torch
                  restatement of nano_ktrans/kernels/cpu_moe.py:491-539) on this
-                 host's cores for the headline; cpu_baselines: every config at
-                 every token count the bench reports (Mixtral T=2048 on a
-                 512-token sample)
-  secondary      other token counts (T=1, 4), the layer from hidden states
+                 host's cores for the headline; cpu_baselines, in short: every other
+                 config and token count the bench reports (Mixtral T=2048 on
+                 a 512-token sample)
+  secondary      in short: other token counts (T=1, 4), the layer from hidden states
                  (router GEMV inside; plus RMSNorm and residual), the tiny
                  fp32 Mixtral-style layer (T=16), the int8 per-channel prefill
                  at T=512/2048/4096 (Zipf-skewed routing), a Mixtral-8x7B-shaped
                  int4 layer (T=1, 16, 2048) and a Qwen1.5-MoE-shaped int8 layer
-                 with its shared expert (T=1, 16, 1024); roofline_alt gives the
-                 other bound's fraction where a shape sits near the ridge
+                 with its shared expert (T=1, 16, 1024)
+The full records go to stderr, one "detail: {...}" line each (roofline_alt there
+gives the other bound's fraction where a shape sits near the ridge).
 """
 import argparse
 import json
@@ -58,6 +59,12 @@ METRIC = "MoE-layer tokens/s + decode µs/layer (Qwen3-30B-A3B shape); % HBM/MFM
 
 def log(*a):
     print(*a, file=sys.stderr, flush=True)
+
+
+def detail(record):
+    """One workload's full record, on stderr (prefixed: the result line is the
+    only line of output that is JSON by itself)."""
+    log("detail:", json.dumps(record))
 
 
 # --------------------------------------------------------------------- problem
@@ -342,7 +349,7 @@ def kernel_form(w, T):
     int8 = 3.5 if w.shared else 4.5
     if avg <= {"int8_per_channel": int8, "int4_g128": 6 if w.I >= 8192 else 8}.get(w.wfmt, 12):
         return "gemv_kernel"
-    # bf16 activations, buffers under 2 GiB (every bench shape): the pipelined kernels
+    # (few large bf16 experts run gemm2_kernel instead, gemm2_bf16_regs: no bench shape)
     return {"int8_per_channel": "gemm2_i8_kernel", "int4_g128": "gemm2_i4_kernel"}.get(w.wfmt, "gemm2_bf16_kernel")
 
 
@@ -713,9 +720,50 @@ def summarize_trace(trace_csv):
 
 # --------------------------------------------------------------------- main
 def _slim(r):
-    keep = ("workload", "tokens", "us_per_layer", "tokens_per_s", "steps", "warmup", "mean_active_experts",
-            "breakdown_us", "roofline", "roofline_alt", "layer_hbm_frac")
-    return {k: v for k, v in r.items() if k in keep}
+    """One workload in the result line, which stays a few KB: readers keep the
+    end of a program's output, 8 KB of it (the full records are on stderr)."""
+    out = {"workload": r["workload"], "tokens": r["tokens"], "us_per_layer": round(r["us_per_layer"], 2),
+           "tokens_per_s": round(r["tokens_per_s"])}
+    if "roofline" in r:
+        f = r["roofline"]
+        vendor = f.get("vendor_gemv") or f.get("vendor_gemm") or {}
+        out["roofline"] = {"kernel": f["kernel"].split(",")[0] + ")", "bound": f["bound"], "frac": f["frac"],
+                           "frac_of_vendor": vendor.get("kernel_frac_of_vendor")}
+    return out
+
+
+def _slim_cpu(c):
+    return {k: c[k] for k in ("workload", "tokens", "value")}
+
+
+def result_line(head, args, res, roofline, cpu_all, secondary):
+    """The program's one line of output: the headline workload in full (cpu_all
+    leads with its CPU baseline), the others in short."""
+    return {
+        "metric": METRIC,
+        "value": round(res["tokens_per_s"], 1),
+        "unit": "tokens/s",
+        "n_gpus": 1,
+        "steps": args.steps,
+        "warmup": args.warmup,
+        "ms_per_step": round(res["ms_per_step"], 5),
+        "higher_is_better": True,
+        "scaling": "weak",
+        "vs_baseline": None,
+        "dtype": "bf16",
+        "data": "synthetic",
+        "config": {"workload": head.name, "tokens": args.tokens, "hidden": head.H, "experts": head.E,
+                   "top_k": head.k, "moe_intermediate": head.I, "weights": "int4 group-128, bf16 scales",
+                   "weight_copies_rotated": args.layers, "parallelism": "single GPU"},
+        "us_per_layer": round(res["us_per_layer"], 2),
+        "mean_active_experts": res["mean_active_experts"],
+        "layer_hbm_frac": round(res["layer_hbm_frac"], 4),
+        "breakdown_us": {k: round(v, 2) for k, v in res["breakdown_us"].items()},
+        "roofline": roofline,
+        "cpu_baseline": cpu_all[0] if cpu_all else None,
+        "cpu_baselines": [_slim_cpu(c) for c in cpu_all[1:]],
+        "secondary": [_slim(r) for r in secondary],
+    }
 
 
 def main():
@@ -756,7 +804,7 @@ def main():
     log(f"headline: {head.name} T={args.tokens}")
     res = bench_workload(head, args.tokens, layers, router, args.steps, args.warmup, dev)
     head_inputs = res.pop("inputs")
-    log(json.dumps({k: v for k, v in res.items()}))
+    detail(res)
     secondary = []
     head_small = {}
     if not args.no_secondary:
@@ -765,7 +813,7 @@ def main():
             r = bench_workload(head, T, layers, router, args.steps, args.warmup, dev)
             head_small[T] = tuple(t.cpu() for t in r.pop("inputs"))
             r["roofline"] = roofline_for(r, "hbm")
-            log(json.dumps(r))
+            detail(r)
             secondary.append(r)
         # the layer from hidden states: the router GEMV [E, H] inside the path
         gate = router.to(torch.bfloat16)
@@ -777,7 +825,7 @@ def main():
         ms = time_graph_hidden(layers, xs, outs, args.steps, args.warmup)
         r = dict(workload=head.name + "_fused_router", tokens=T, us_per_layer=ms * 1e3,
                  tokens_per_s=T / (ms * 1e-3), steps=args.steps, warmup=args.warmup)
-        log(json.dumps(r))
+        detail(r)
         secondary.append(r)
         # the decoder layer's MoE half: residual + MoE(RMSNorm(hidden)), router inside
         norm_w = (1.0 + 0.1 * torch.randn(head.H, generator=torch.Generator().manual_seed(3))).to(dev)
@@ -785,20 +833,19 @@ def main():
         ms = time_graph_hidden(layers, xs, outs, args.steps, args.warmup, call=fwd)
         r = dict(workload=head.name + "_decoder_block", tokens=T, us_per_layer=ms * 1e3,
                  tokens_per_s=T / (ms * 1e-3), steps=args.steps, warmup=args.warmup)
-        log(json.dumps(r))
+        detail(r)
         secondary.append(r)
     del layers
     torch.cuda.empty_cache()
-    cpu = None
     if do_cpu:
         log(f"cpu baseline: {head.name} T={args.tokens}")
         cpu = cpu_baseline(head, args.tokens, src, *head_inputs)
-        log(json.dumps(cpu))
+        detail(cpu)
         cpu_all.append(cpu)
         for T, inp in head_small.items():
             log(f"cpu baseline: {head.name} T={T}")
             c = cpu_baseline(head, T, src, *inp)
-            log(json.dumps(c))
+            detail(c)
             cpu_all.append(c)
     del src
     if not args.no_secondary:
@@ -829,7 +876,7 @@ def main():
                 r["roofline"] = roofline_for(r, bounds[0])
                 if len(bounds) > 1:
                     r["roofline_alt"] = roofline_for(r, bounds[1])
-                log(json.dumps(r))
+                detail(r)
                 secondary.append(r)
             del lays
             torch.cuda.empty_cache()
@@ -837,34 +884,10 @@ def main():
                 for T, sample in cpu_runs:
                     log(f"cpu baseline: {w.name} T={T} sample={sample}")
                     c = cpu_baseline(w, T, wsrc, *inputs[T], sample=sample)
-                    log(json.dumps(c))
+                    detail(c)
                     cpu_all.append(c)
             del wsrc
-    line = {
-        "metric": METRIC,
-        "value": round(res["tokens_per_s"], 1),
-        "unit": "tokens/s",
-        "n_gpus": 1,
-        "steps": args.steps,
-        "warmup": args.warmup,
-        "ms_per_step": round(res["ms_per_step"], 5),
-        "higher_is_better": True,
-        "scaling": "weak",
-        "vs_baseline": None,
-        "dtype": "bf16",
-        "data": "synthetic",
-        "config": {"workload": head.name, "tokens": args.tokens, "hidden": head.H, "experts": head.E,
-                   "top_k": head.k, "moe_intermediate": head.I, "weights": "int4 group-128, bf16 scales",
-                   "weight_copies_rotated": args.layers, "parallelism": "single GPU"},
-        "us_per_layer": round(res["us_per_layer"], 2),
-        "mean_active_experts": res["mean_active_experts"],
-        "layer_hbm_frac": round(res["layer_hbm_frac"], 4),
-        "breakdown_us": {k: round(v, 2) for k, v in res["breakdown_us"].items()},
-        "roofline": roofline_for(res, "hbm"),
-        "cpu_baseline": cpu,
-        "cpu_baselines": cpu_all,
-        "secondary": [_slim(r) for r in secondary],
-    }
+    line = result_line(head, args, res, roofline_for(res, "hbm"), cpu_all, secondary)
     print(json.dumps(line), flush=True)
 
 
