@@ -387,7 +387,8 @@ COUNTERS_MD = os.path.join(ROOT, "profiles", "pmc_moe_layer_counters.md")
 def counter_table():
     """Per-launch HBM traffic and matrix-core counters of the expert GEMMs, measured
     with rocprofv3 --pmc on nkt_probe (profiles/pmc_moe_layer_counters.md), keyed
-    (probe workload, tokens, phase) -> {"traffic": bytes, "mfma_util": %}."""
+    (probe workload, tokens, phase) -> {"kernel": name with template arguments,
+    "traffic": bytes, "mfma_util": %}."""
     try:
         text = open(COUNTERS_MD).read()
     except OSError:
@@ -402,11 +403,25 @@ def counter_table():
         if key.count(":") != 2:
             continue
         try:
-            out[key] = {"traffic": float(cells[5]),
+            out[key] = {"kernel": cells[1].strip("`"), "traffic": float(cells[5]),
                         "mfma_util": float(cells[6]) if cells[6] not in ("", "-") else None}
         except (ValueError, IndexError):
             pass
     return out
+
+
+def counters_apply(row, kernel, phase):
+    """Whether a counter row was taken on this kernel: its name and the template
+    arguments that identify its present form (gemv_kernel<WF, PHASE, 7 more>,
+    gemm_kernel<6 and PHASE>, gemm2_i8_kernel<PHASE, F16>, gemm2_i4_kernel<PHASE,
+    4 or 8 waves>, gemm2_bf16_kernel<PHASE>, gemm2_kernel<PHASE>)."""
+    import re
+
+    ph = 0 if phase == "gate_up" else 1
+    form = {"gemv_kernel": rf"\d, {ph}(, \w+){{7}}", "gemm_kernel": rf"\d, \d+, \d, \d, {ph}, \d+, \d",
+            "gemm2_i8_kernel": rf"{ph}, (true|false)", "gemm2_i4_kernel": rf"{ph}, [48]",
+            "gemm2_bf16_kernel": f"{ph}", "gemm2_kernel": f"{ph}"}[kernel]
+    return re.fullmatch(rf"nkt::{kernel}<{form}>", row.get("kernel", "")) is not None
 
 
 _CEILINGS = {}
@@ -491,6 +506,8 @@ def roofline_for(res, bound=None):
     sec = d["us"] * 1e-6
     name = f"{d['kernel']} ({k}, {res['wfmt']}, T={res['tokens']})"
     row = counter_table().get(f"{res['probe']}:{res['tokens']}:{k}", {})
+    if not counters_apply(row, d["kernel"], k):
+        row = {}  # counters of another kernel than the one timed
     traffic = row.get("traffic")
     if bound == "hbm":
         achieved = d["bytes"] / sec / 1e9

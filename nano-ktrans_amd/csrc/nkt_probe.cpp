@@ -6,7 +6,7 @@
 // With "layer" each step is one nkt_moe_forward call (the layer's own launch
 // sequence); otherwise the stage entry points run one by one.
 //
-// workload: qwen3_int4 | qwen3_int8 | mixtral_int4 | qwen15_int8 | tiny_f32.
+// workload: qwen3_int4 | qwen3_int8 | qwen3_bf16 | mixtral_int4 | qwen15_int8 | tiny_f32.
 // It first runs a calibration kernel of known traffic (fp32 negate over
 // 256 MiB in and out, three launches), then `copies` distinct weight copies of
 // the layer (quantized projections packed by nkt_moe_pack_weight from random
@@ -95,6 +95,7 @@ struct Workload {
 static const Workload kWorkloads[] = {
     {"qwen3_int4", 2048, 128, 8, 768, 0, NKT_WEIGHT_INT4_G128, NKT_DTYPE_BF16, NKT_ROUTE_SOFTMAX | NKT_ROUTE_RENORM, 0.f},
     {"qwen3_int8", 2048, 128, 8, 768, 0, NKT_WEIGHT_INT8_PC, NKT_DTYPE_BF16, NKT_ROUTE_SOFTMAX | NKT_ROUTE_RENORM, 1.1f},
+    {"qwen3_bf16", 2048, 128, 8, 768, 0, NKT_WEIGHT_BF16, NKT_DTYPE_BF16, NKT_ROUTE_SOFTMAX | NKT_ROUTE_RENORM, 0.f},
     {"mixtral_int4", 4096, 8, 2, 14336, 0, NKT_WEIGHT_INT4_G128, NKT_DTYPE_BF16, 0u, 0.f},
     {"qwen15_int8", 2048, 60, 4, 1408, 5632, NKT_WEIGHT_INT8_PC, NKT_DTYPE_BF16, NKT_ROUTE_SOFTMAX, 0.f},
     {"tiny_f32", 256, 8, 2, 512, 0, NKT_WEIGHT_F32, NKT_DTYPE_F32, NKT_ROUTE_SOFTMAX | NKT_ROUTE_RENORM, 0.f},

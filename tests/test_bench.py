@@ -40,3 +40,18 @@ def test_result_line_fits_the_kept_end_of_the_output(capsys):
     bench.detail(r)
     for out in capsys.readouterr().err.splitlines():
         assert not out.startswith("{")
+
+
+def test_counter_rows_join_the_kernel_that_they_were_taken_on():
+    """A counter row goes beside a kernel's time only if it was taken on that
+    kernel's present form; every committed row is."""
+    table = bench.counter_table()
+    assert table
+    for key, row in table.items():
+        phase = key.split(":")[2].replace("shared_", "").replace("_layer_call", "")
+        name = row["kernel"].split("::")[1].split("<")[0]
+        assert bench.counters_apply(row, name, phase), key
+        assert not bench.counters_apply(row, name, "down" if phase == "gate_up" else "gate_up")
+    assert not bench.counters_apply({"kernel": "nkt::gemm2_i4_kernel<0, false>"}, "gemm2_i4_kernel", "gate_up")
+    assert not bench.counters_apply({"kernel": "nkt::gemm2_kernel<1, 0, 8>"}, "gemm2_kernel", "gate_up")
+    assert not bench.counters_apply({}, "gemv_kernel", "gate_up")
