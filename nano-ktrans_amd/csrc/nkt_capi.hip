@@ -197,8 +197,9 @@ WsLayout ws_layout(const Handle* h, int T) {
   // measured faster at every such T (Qwen1.5-MoE int8 T = 96 / 128 / 192 /
   // 256 146 / 150 / 169 / 190 -> 129 / 133 / 137 / 138 us per layer), while
   // inside the decode range the chunk tiles win (T = 48 / 64 121 / 132
-  // against 140 / 147).  Without the int8 / int4 prefill pipelines the
-  // decode form's split-K grid keeps it up to kSharedDecodeMaxTokens.
+  // against 140 / 147).  bf16 and fp32 keep the decode form's split-K grid up
+  // to kSharedDecodeMaxTokens (bf16's prefill pipeline is younger than that
+  // line and not measured there).
   const bool shared_prefill = (h->wf == WF_I8 || h->wf == WF_I4) && prefill_form_ok(h, true) && L.bm != kTileSrcCols;
   L.bm_shared = (T <= kSharedDecodeMaxTokens && h->Is > 0 && !shared_prefill &&
                  gemv_supported(h->wf, PHASE_GATE_UP, 2 * h->Is, h->H, h->Is) &&

@@ -354,7 +354,9 @@ __global__ void __launch_bounds__(NW * 64) gemm_kernel(GemmArgs a) {
 // prefill form wins: Qwen3 T = 192 107.8 -> 99.1 us, Mixtral T = 48 222 ->
 // 197, T = 64 285 -> 225) -- 6 for experts of I >= 8192, whose decode down
 // takes the long-K ring (Mixtral, T = 28 / 32: 189.6 / 194.8 -> 183.9 /
-// 180.5 us; level at 6, decode ahead at 5), others 12.
+// 180.5 us; level at 6, decode ahead at 5), others 12.  (int4's and bf16's
+// lines come from the prefill kernels before the four-wave int4 form and the
+// bf16 pipeline, 7 - 20 % and 3 - 12 % slower; not measured again since.)
 double decode_form_max_avg(int wf, int I, bool shared) {
   return wf == WF_I8 ? (shared ? 3.5 : 4.5) : wf == WF_I4 ? (I >= 8192 ? 6.0 : 8.0) : 12.0;
 }

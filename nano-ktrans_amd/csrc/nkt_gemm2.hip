@@ -19,7 +19,7 @@
 //     its reads share the L2 better (gemm2_bf16_regs) and experts of 2 GiB
 //     and more.  (All address one expert's projection with 32-bit offsets;
 //     a handle holds none of 4 GiB or more.)
-// The pipelines also hold copies that compute only the first 16 / 32
+// The pipelines also hold copies that compute only the first 16 / 32 / 48
 // positions of a tile, taken by tiles with no more (an expert's last or
 // only tile): the matrix-core work of empty column tiles is skipped, and an
 // expert's only tile loads its weights non-temporally.
@@ -521,9 +521,10 @@ __global__ void __launch_bounds__(512, 2) gemm2_kernel(GemmArgs a, int n_slabs, 
 }
 
 // ---------------------------------------------------------------------------
-// int8 (and bf16) weights, three-stage pipeline.  Same tile, waves, work order, MFMA
-// sequence and epilogue as gemm2_kernel<WF_I8, ...> (so the results are the
-// same bit for bit); K advances in 64-wide stages:
+// int8 (and bf16) weights, three-stage pipeline: 4 waves of four 16-row
+// tiles; an output's 32-wide MFMA steps add in ascending K (bf16 gives
+// gemm2_kernel's bits).  K advances in 64-wide stages (int8's numbers; bf16
+// has two blocks per row tile and stage, so 10 loads in place of 6):
 //   * weights: each wave's own 4 row tiles, one 1 KiB block (16 rows x 64 K,
 //     lane l's MFMA fragments at 16 l) per row tile, loaded by buffer loads
 //     straight into a ring of three register stages (the weights are private
@@ -788,8 +789,8 @@ __global__ void __launch_bounds__(256, 2) gemm2_i8_kernel(GemmArgs a, int n_slab
 // copies (launch_gemm2 still takes it for few large experts: gemm2_bf16_regs).
 // Measured, gemm2_kernel -> this (Qwen3 bf16, us per layer): T = 200 / 700 /
 // 1000 / 2000 / 4096 230 / 275 / 282 / 375 / 606 -> 207 / 249 / 277 / 356 /
-// 535; the full tile's nt copy (an expert's only tile of 49 - 64 positions)
-// T = 850 / 1000 265 / 285 -> 250 / 277.
+// 535; the nt copy over all four column tiles (an expert's only tile of 49 -
+// 63 positions) T = 850 / 1000 265 / 285 -> 250 / 277.
 template <int PHASE>
 __global__ void __launch_bounds__(256, 2) gemm2_bf16_kernel(GemmArgs a, int n_slabs, int sg) {
   gemm2_stage64<WF_BF16, PHASE, false>(a, n_slabs, sg);
@@ -879,8 +880,11 @@ bool gemm2_supported(int wf, int phase, int N, int K, int I) {
 // Both forms, whatever the launch, sum an output's K groups in ascending
 // order and h's group sums over 16-column tiles in ascending order, so an
 // int4 prefill row has the same bits in every batch.
-// What bounds it: neither HBM nor one unit, but the waits a stage's barrier
-// and an item's start and end leave.  Four waves of 64 rows read each token
+// What bounds it: neither HBM nor one unit.  By counters its waves issue in 32
+// - 41 % of their cycles, wait for a free unit in 34 - 42 % and for loads or a
+// stage's barrier in 21 - 32 % (Mixtral T = 2048, Qwen3 T = 203 / 2048), the
+// matrix cores busy 47 / 39 % of Mixtral's gate_up / down; at least 98.6 % of
+// the instruction fetches hit.  Four waves of 64 rows read each token
 // fragment from LDS half as often as eight waves of 32 and fit two
 // workgroups per CU (251 VGPRs at 2 waves per SIMD), so one computes while
 // the other waits: at Mixtral T = 2000 gate_up 853 us (four) against 999

@@ -256,10 +256,11 @@ hipError_t launch_group_sums(const void* x, int rows, int K, float* out, hipStre
 // (x16, same layout) and 1 / scale per row (xinv); K <= 4096
 hipError_t launch_prep_f16(const void* x, int rows, int K, float* sums, uint16_t* x16, float* xinv,
                            hipStream_t stream);
-// K1 for T tokens (bf16 logits, as launch_route) and launch_prep_f16 of
+// K1 for T tokens (bf16 logits, as launch_route) and launch_group_sums of
 // rows rows of x in one launch.
 hipError_t launch_route_sums(const void* logits, int T, int E, int k, unsigned flags, int32_t* ids, float* w,
                              const void* x, int rows, int K, float* sums, hipStream_t stream);
+// the same with launch_prep_f16 of those rows
 hipError_t launch_route_prep_f16(const void* logits, int T, int E, int k, unsigned flags, int32_t* ids, float* w,
                                  const void* x, int rows, int K, float* sums, uint16_t* x16, float* xinv,
                                  hipStream_t stream);
