@@ -170,7 +170,9 @@ int nkt_moe_route_given(void* handle, const int64_t* topk_ids, const float* topk
 /* K3: grouped SwiGLU expert GEMM for the routed experts (needs a prior
  * nkt_moe_route on the same workspace).  Replaces the per-expert loop
  * nano_ktrans/layers/hybrid_moe.py:3501-3533 / expert_mlp.py:20-41 and
- * nano_ktrans/kernels/cpu_moe.py:419-450.  Writes NKT_WS_H and NKT_WS_Y. */
+ * nano_ktrans/kernels/cpu_moe.py:419-450.  Writes NKT_WS_H and NKT_WS_Y.
+ * hidden_states here and below: 16-byte aligned (int4's prefill form moves
+ * 16-byte pieces of its rows straight into LDS). */
 int nkt_moe_experts(void* handle, const void* hidden_states, int num_tokens, void* workspace,
                     size_t workspace_bytes, void* stream, char* err, size_t err_len);
 

@@ -836,9 +836,10 @@ bool gemm2_i8_pipeline(const GemmArgs& a, int wf) {
   return wf == WF_I8 && a.in_bytes <= (int64_t)kI8Skip && (int64_t)a.N * a.K <= (int64_t)kI8Skip;
 }
 
-// the same for bf16 weights (bf16 activations)
+// the same for bf16 weights (bf16 activations, 16-byte aligned for the
+// direct-to-LDS loads; gemm2_kernel's global loads take any address)
 bool gemm2_bf16_pipeline(const GemmArgs& a, int wf) {
-  return wf == WF_BF16 && a.in_bytes > 0 && a.in_bytes <= (int64_t)kI8Skip && a.w_expert_bytes < (int64_t)kBf16Skip;
+  return wf == WF_BF16 && (uintptr_t)a.in % 16 == 0 && a.in_bytes > 0 && a.in_bytes <= (int64_t)kI8Skip && a.w_expert_bytes < (int64_t)kBf16Skip;
 }
 
 // the int4 pipeline addresses weights, scales, group sums and activations

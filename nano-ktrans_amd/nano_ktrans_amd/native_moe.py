@@ -246,6 +246,11 @@ class NativeMoE:
             raise ValueError(f"{name} has {t.shape[1]} columns, expected {cols}")
         return t.contiguous()
 
+    def _check_hidden(self, hidden_states: torch.Tensor) -> torch.Tensor:
+        x = self._check_input(hidden_states, self.hidden_size, "hidden_states")
+        # the prefill kernels move 16-byte pieces of the rows straight into LDS
+        return x if x.data_ptr() % 16 == 0 else x.clone()
+
     def route(self, router_logits: torch.Tensor):
         """K1 + K2.  Returns (ids int32 [T,k], weights fp32 [T,k], counts [E], offsets [E+1],
         perm [T*k], inv [T*k]) as views of the workspace."""
@@ -305,7 +310,7 @@ class NativeMoE:
         """The layer on the caller's routing: out[t] = sum over the token's slots (ascending expert id)
         of topk_weights[t, j] * expert_{topk_ids[t, j]}(x_t), plus the gated shared expert when the
         layer has one; experts marked non-resident (``set_residency``) add nothing."""
-        x = self._check_input(hidden_states, self.hidden_size, "hidden_states")
+        x = self._check_hidden(hidden_states)
         T = x.shape[0]
         ids, w = self._check_routing(topk_ids, topk_weights, T)
         if out is None:
@@ -342,7 +347,7 @@ class NativeMoE:
     def route_hidden(self, hidden_states: torch.Tensor):
         """Router GEMV + K1 + K2 from hidden states (after ``load_router``).  Returns
         (router_logits bf16 [T, E], ids, weights, counts, offsets, perm, inv) as views."""
-        x = self._check_input(hidden_states, self.hidden_size, "hidden_states")
+        x = self._check_hidden(hidden_states)
         T = x.shape[0]
         ws = self.workspace(T)
         with torch.cuda.device(self.device):
@@ -362,7 +367,7 @@ class NativeMoE:
         """K3 after ``route``: returns h [T*k, I] (act dtype) by position and y [T*k, H] (fp32), whose row is
         the pair t*k + slot in the decode form (T*k / E up to 4.5 for int8 weights (3.5 with a shared
         expert), 8 for int4 (6 for I >= 8192), 12 for the others) and the position otherwise."""
-        x = self._check_input(hidden_states, self.hidden_size, "hidden_states")
+        x = self._check_hidden(hidden_states)
         T = x.shape[0]
         ws = self.workspace(T)
         with torch.cuda.device(self.device):
@@ -376,7 +381,8 @@ class NativeMoE:
         """One K3 launch after ``route``: phase 0 gate_up + SwiGLU, phase 1 down."""
         xp = None
         if phase == 0:
-            xp = self._check_input(hidden_states, self.hidden_size, "hidden_states").data_ptr()
+            x = self._check_hidden(hidden_states)  # a copy of it lives until the launch is queued
+            xp = x.data_ptr()
         ws = self.workspace(num_tokens)
         with torch.cuda.device(self.device):
             self.err.check(self.lib.nkt_moe_experts_phase(self.handle, phase, xp, num_tokens, ws.data_ptr(),
@@ -389,7 +395,8 @@ class NativeMoE:
         (events created with enable_timing=True) at the kernel's own start and end."""
         xp = None
         if phase == 0:
-            xp = self._check_input(hidden_states, self.hidden_size, "hidden_states").data_ptr()
+            x = self._check_hidden(hidden_states)  # a copy of it lives until the launch is queued
+            xp = x.data_ptr()
         ws = self.workspace(num_tokens)
         with torch.cuda.device(self.device):
             self.err.check(self.lib.nkt_moe_experts_phase_timed(
@@ -399,7 +406,7 @@ class NativeMoE:
 
     def shared(self, hidden_states: torch.Tensor):
         """K4 + K3 on the shared expert: returns (gate fp32 [T], y_shared fp32 [T, H])."""
-        x = self._check_input(hidden_states, self.hidden_size, "hidden_states")
+        x = self._check_hidden(hidden_states)
         T = x.shape[0]
         ws = self.workspace(T)
         with torch.cuda.device(self.device):
@@ -449,7 +456,7 @@ class NativeMoE:
 
     def forward_hidden(self, hidden_states: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The whole layer from hidden states (router GEMV fused; after ``load_router``)."""
-        x = self._check_input(hidden_states, self.hidden_size, "hidden_states")
+        x = self._check_hidden(hidden_states)
         T = x.shape[0]
         if out is None:
             out = torch.empty(T, self.hidden_size, dtype=self.act_dtype, device=self.device)
@@ -466,7 +473,7 @@ class NativeMoE:
                       out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The decoder layer's MoE half: hidden + MoE(RMSNorm(hidden)) with the fused
         router (after ``load_router``); the RMSNorm output stays in NKT_WS_NORMED."""
-        x = self._check_input(hidden_states, self.hidden_size, "hidden_states")
+        x = self._check_hidden(hidden_states)
         T = x.shape[0]
         w = norm_weight.to(self.act_dtype).to(self.device).reshape(-1).contiguous()
         if w.numel() != self.hidden_size:
@@ -486,7 +493,7 @@ class NativeMoE:
     def forward(self, hidden_states: torch.Tensor, router_logits: torch.Tensor,
                 out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The whole layer; returns [T, H] in the activation dtype."""
-        x = self._check_input(hidden_states, self.hidden_size, "hidden_states")
+        x = self._check_hidden(hidden_states)
         logits = self._check_input(router_logits, self.num_experts, "router_logits")
         T = x.shape[0]
         if logits.shape[0] != T:
@@ -507,7 +514,7 @@ class NativeMoE:
         """``forward`` through nkt_moe_forward_noalloc: the library's static
         per-GPU scratch replaces the workspace, so the call allocates nothing
         (``out`` is the caller's).  Calls that overlap on one GPU race."""
-        x = self._check_input(hidden_states, self.hidden_size, "hidden_states")
+        x = self._check_hidden(hidden_states)
         logits = self._check_input(router_logits, self.num_experts, "router_logits")
         T = x.shape[0]
         if logits.shape[0] != T:

@@ -122,3 +122,23 @@ def test_bf16_expert_past_2_gib(gpu_device):
         a, b = x.float() @ gate[i:i + 16384].float().T, x.float() @ up[i:i + 16384].float().T
         ref += (torch.nn.functional.silu(a) * b) @ down[:, i:i + 16384].float().T
     compare(out.float().cpu().numpy(), ref.cpu().numpy(), cfg)
+
+
+@pytest.mark.parametrize("wfmt", ["int4_g128", "bf16", "int8_per_channel"])
+def test_rows_at_any_address(gpu_device, wfmt):
+    """hidden_states that start between 16-byte boundaries (a contiguous view
+    one element into its storage) give the bits of an aligned copy, in the
+    decode form (T = 3) and the prefill form."""
+    cfg = replace(CONFIGS["qwen3_int4"], name=f"offset_{wfmt}", H=512, I=384, E=2, k=2, wfmt=wfmt)
+    layer = build_layer(cfg, device="cuda")
+    native = native_layer(layer, torch.device("cuda"))
+    for T in (3, 33, 130):
+        x, logits = build_inputs(layer, T, seed=T, device="cuda")
+        store = torch.zeros(x.numel() + 16, dtype=x.dtype, device="cuda")
+        view = store[1:1 + x.numel()].view(T, cfg.H)
+        view.copy_(x)
+        assert view.data_ptr() % 16 == 2
+        aligned = native.forward(x, logits).clone()
+        offset = native.forward(view, logits)
+        torch.cuda.synchronize()
+        assert torch.equal(aligned, offset), f"T = {T}"
